@@ -161,6 +161,21 @@ int nf_adaln_bwd_reduce(void *workspace, size_t workspace_bytes,
                         int dt_weight, int dt_scale, int dt_shift,
                         void *stream);
 
+/* The whole adaLN seam backward in one call: the results of nf_adaln_bwd and
+ * nf_adaln_bwd_reduce (same arguments, outputs each NULL where not wanted),
+ * with a workspace of nf_adaln_bwd_workspace(M, N, T) bytes.  With many
+ * samples it runs without partial rows per sample (the sums differ from the
+ * two calls' by fp32 rounding only); fixed orders, no atomics. */
+int nf_adaln_bwd_full(const void *dh_up, const void *dout, const void *x,
+                      int64_t ld_x, const void *y, int64_t ld_y,
+                      const void *gate, int64_t ld_gate, const void *weight,
+                      const void *scale, int64_t ld_scale, const float *rstd,
+                      void *dx, void *dy, void *dgate, void *dweight,
+                      void *dscale, void *dshift, void *workspace,
+                      size_t workspace_bytes, int64_t M, int64_t N, int64_t T,
+                      int dt_x, int dt_y, int dt_gate, int dt_weight,
+                      int dt_scale, int dt_shift, void *stream);
+
 /* Size of the static device buffer nf_adaln_bwd_noalloc keeps its partial
  * rows in (one per GPU, held until the process ends). */
 #define NF_ADALN_SCRATCH_BYTES ((size_t)16 << 20)

@@ -13,7 +13,10 @@ namespace adaln {
   extern template int fwd_v<TX, TY>(const FwdArgs &, const Plan &, bool,     \
                                     hipStream_t);                            \
   extern template int bwd_v<TX, TY>(const BwdArgs &, const Plan &, bool,     \
-                                    hipStream_t);
+                                    hipStream_t);                            \
+  extern template int bwd_walk<TX, TY>(const BwdArgs &, const WalkOut &,     \
+                                       const Plan &, const WalkPlan &,       \
+                                       hipStream_t);
 NF_ADALN_EXTERN(float, float)
 NF_ADALN_EXTERN(bf16, bf16)
 NF_ADALN_EXTERN(f16, f16)
@@ -255,6 +258,27 @@ __global__ __launch_bounds__(kRcThreads) void adaln_reduce_kernel(ReduceArgs p) 
   store_dyn(out, dt, (int64_t)b * N + c, wc * acc);
 }
 
+// dweight from the sample-walking backward: the `rows` [N] fp32 rows its
+// blocks wrote, added in a fixed order (row group k of a block takes rows k,
+// k + 32, ..., then the 32 groups in order), one block per 32-column slice.
+__global__ __launch_bounds__(kRcThreads) void adaln_dweight_kernel(const float *wpart, int rows,
+                                                                   int N, void *dweight,
+                                                                   int dt_weight) {
+  __shared__ float red[kRcGroups][kRcCols];
+  const int t = threadIdx.x, lane = t % kRcLanes, g = t / kRcLanes;
+  const int col = blockIdx.x * kRcCols + 4 * lane;
+  put4(&red[g][4 * lane], sum_rows<true>(wpart, N, g, kRcGroups, rows, col, N));
+  __syncthreads();
+  const int cc = blockIdx.x * kRcCols + t;
+  if (t >= kRcCols || cc >= N) return;
+  float x[kRcGroups], a = 0.f;
+#pragma unroll
+  for (int k = 0; k < kRcGroups; ++k) x[k] = red[k][t];
+#pragma unroll
+  for (int k = 0; k < kRcGroups; ++k) a += x[k];
+  store_dyn(dweight, dt_weight, cc, a);
+}
+
 }  // namespace adaln
 }  // namespace nf
 
@@ -385,6 +409,55 @@ extern "C" int nf_adaln_bwd_reduce(void *workspace,
   else
     adaln_reduce_kernel<false><<<(unsigned)grid, kRcThreads, 0, s>>>(r);
   return check_launch("nf_adaln_bwd_reduce");
+}
+
+// Both passes of the backward in one call: the sample-walking kernel where its
+// rule holds (see make_walk_plan) and every row is whole aligned vectors,
+// else the row kernel and the reduction.
+extern "C" int nf_adaln_bwd_full(const void *dh_up, const void *dout, const void *x,
+                                 int64_t ld_x, const void *y, int64_t ld_y,
+                                 const void *gate, int64_t ld_gate, const void *weight,
+                                 const void *scale, int64_t ld_scale, const float *rstd,
+                                 void *dx, void *dy, void *dgate, void *dweight, void *dscale,
+                                 void *dshift, void *workspace, size_t workspace_bytes_given,
+                                 int64_t M, int64_t N, int64_t T, int dt_x, int dt_y,
+                                 int dt_gate, int dt_weight, int dt_scale, int dt_shift,
+                                 void *stream) {
+  if (int e = check_shape("nf_adaln_bwd_full", M, N, T)) return e;
+  if (!is_dtype(dt_gate) || !is_dtype(dt_weight) || !is_dtype(dt_scale) || !is_dtype(dt_shift))
+    return set_error(NF_ERR_DTYPE, "nf_adaln_bwd_full: bad conditioning dtype");
+  const Plan pl = M > 0 ? make_plan(M, N, T) : Plan{};
+  const WalkPlan w = M > 0 ? make_walk_plan(pl, N, T) : WalkPlan{};
+  const bool any = dgate || dweight || dscale || dshift;
+  if (w.use && any && x && y && gate && weight && scale && rstd && dx && dy && workspace &&
+      workspace_bytes_given >= workspace_bytes(pl, N) && ld_x >= N && ld_y >= N &&
+      ld_gate >= 0 && ld_scale >= 0 && ld_x % 8 == 0 && ld_y % 8 == 0 && ld_gate % 8 == 0 &&
+      ld_scale % 8 == 0 && aligned16(x) && aligned16(y) && aligned16(gate) &&
+      aligned16(weight) && aligned16(scale) && aligned16(dx) && aligned16(dy) &&
+      aligned16(workspace) && aligned16(dh_up) && aligned16(dout) && aligned16(dgate) &&
+      aligned16(dscale) && aligned16(dshift)) {
+    BwdArgs a{dh_up, dout, x, y, gate, weight, scale, rstd, dx, dy,
+              nullptr, ld_x, ld_y, ld_gate, ld_scale,
+              M, T, (int)N, 1, (int)T, dt_gate, dt_weight, dt_scale};
+    float *wpart = static_cast<float *>(workspace);  // blocks <= B rows of N
+    const WalkOut o{dgate, dscale, dshift, wpart, dt_shift, pl.B, w.per_unit};
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    if (int e = dispatch_xy(dt_x, dt_y, "nf_adaln_bwd_full", [&](auto tx, auto ty) {
+          return bwd_walk<decltype(tx), decltype(ty)>(a, o, pl, w, s);
+        }))
+      return e;
+    if (!dweight) return NF_OK;
+    adaln_dweight_kernel<<<(unsigned)((N + kRcCols - 1) / kRcCols), kRcThreads, 0, s>>>(
+        wpart, (int)w.blocks, (int)N, dweight, dt_weight);
+    return check_launch("nf_adaln_bwd_full");
+  }
+  if (int e = nf_adaln_bwd(dh_up, dout, x, ld_x, y, ld_y, gate, ld_gate, weight, scale, ld_scale,
+                           rstd, dx, dy, workspace, workspace_bytes_given, M, N, T, dt_x, dt_y,
+                           dt_gate, dt_weight, dt_scale, stream))
+    return e;
+  return nf_adaln_bwd_reduce(workspace, workspace_bytes_given, weight, scale, ld_scale, dgate,
+                             dweight, dscale, dshift, M, N, T, dt_gate, dt_weight, dt_scale,
+                             dt_shift, stream);
 }
 
 // ---------------------------------------------------------------------------

@@ -365,33 +365,38 @@ __global__ __launch_bounds__((FwdShape<WPR, fwd_min_block<K>()>::BLK)) void adal
 // backward: per-row gradients + per-block partial rows
 // ---------------------------------------------------------------------------
 
-// Sum one accumulator over the G row groups of the block (group order
-// 0, 1, ..., G-1) and store the result row.  All threads must call it.
-template <int K, int G, int R, bool VEC>
-__device__ __forceinline__ void combine_store(float (&acc)[K][8], float *comb,
-                                              int g, int rt, float *dst,
-                                              int N) {
+// Sum one accumulator over the G row groups of the block into group 0's
+// registers (group order 0, 1, ..., G-1).  All threads must call it.
+template <int K, int G, int R>
+__device__ __forceinline__ void combine_groups_lds(float (&acc)[K][8], float *comb, int g,
+                                                   int rt) {
   constexpr int kRowElems = R * K * 8;
-  if constexpr (G > 1) {
-    if (g > 0) {
+  if (g > 0) {
+#pragma unroll
+    for (int k = 0; k < K; ++k)
+#pragma unroll
+      for (int i = 0; i < 8; ++i)
+        comb[(g - 1) * kRowElems + (k * R + rt) * 8 + i] = acc[k][i];
+  }
+  __syncthreads();
+  if (g == 0) {
+#pragma unroll
+    for (int gg = 1; gg < G; ++gg)
 #pragma unroll
       for (int k = 0; k < K; ++k)
 #pragma unroll
         for (int i = 0; i < 8; ++i)
-          comb[(g - 1) * kRowElems + (k * R + rt) * 8 + i] = acc[k][i];
-    }
-    __syncthreads();
-    if (g == 0) {
-#pragma unroll
-      for (int gg = 1; gg < G; ++gg)
-#pragma unroll
-        for (int k = 0; k < K; ++k)
-#pragma unroll
-          for (int i = 0; i < 8; ++i)
-            acc[k][i] += comb[(gg - 1) * kRowElems + (k * R + rt) * 8 + i];
-    }
-    __syncthreads();
+          acc[k][i] += comb[(gg - 1) * kRowElems + (k * R + rt) * 8 + i];
   }
+  __syncthreads();
+}
+
+// combine_groups_lds, then the result row stored by group 0.
+template <int K, int G, int R, bool VEC>
+__device__ __forceinline__ void combine_store(float (&acc)[K][8], float *comb,
+                                              int g, int rt, float *dst,
+                                              int N) {
+  if constexpr (G > 1) combine_groups_lds<K, G, R>(acc, comb, g, rt);
   if (g == 0) {
 #pragma unroll
     for (int k = 0; k < K; ++k) {
@@ -722,6 +727,224 @@ __global__ __launch_bounds__((BwdShape<WPR>::BLK)) void adaln_bwd_pipe_kernel(Bw
 }
 
 // ---------------------------------------------------------------------------
+// backward over many samples: a block walks whole samples, so each sample's
+// dgate / dscale / dshift are finished where its rows are and go out in their
+// own types, and the block's share of dweight = sum_b (1 + scale_b) A_b stays
+// in registers until one [N] fp32 row per block is written.  What it replaces
+// is bound by the partial rows: with one block per sample the row kernel
+// writes 12 N bytes a sample and the reduction reads them back, its dweight
+// blocks 32 samples a round, ~1.7 us a round (x fp32, y bf16 [2048, 6, 384]:
+// 27 + 110 us; here 20 us and 4 for the dweight rows).
+// COOP: the G row groups of a block share each sample's rows (group g takes
+// rows g, g + G, ...) and combine in LDS in group order; otherwise each row
+// group walks samples of its own and nothing is exchanged but the row sums.
+// Either way the units of a block (groups, or the block itself) hold
+// consecutive samples, so the rows are one flattened run per unit: the next
+// row's loads are issued before the current row's math and stores (two
+// register buffers in turn) also across a sample's end, and the next sample's
+// conditioning is loaded while the current sample's rows are worked on.  All
+// row groups step through rows and samples together (row_sum synchronises);
+// a group past its rows or samples steps along without touching memory.
+// ---------------------------------------------------------------------------
+struct WalkOut {
+  void *dgate;     // [B, N] each, or null
+  void *dscale;
+  void *dshift;
+  float *wpart;    // [gridDim.x, N]
+  int dt_shift;
+  int64_t B;
+  int per_unit;    // consecutive samples per unit
+};
+
+constexpr int kWalkMinBlock = 256;
+
+template <typename TX, typename TY, int K, int WPR, bool COOP, bool NT, bool NTL>
+__global__ __launch_bounds__((BwdShape<WPR, kWalkMinBlock>::BLK)) void adaln_bwd_walk_kernel(
+    BwdArgs p, WalkOut o) {
+  using S = BwdShape<WPR, kWalkMinBlock>;
+  constexpr int GS = COOP ? S::G : 1;  // row groups per sample
+  __shared__ float red[S::G * WPR];
+  __shared__ float comb[S::G > 1 ? (S::G - 1) * S::R * K * 8 : 1];
+  const int g = threadIdx.x / S::R;
+  const int rt = threadIdx.x % S::R;
+  const int64_t b0 = (COOP ? (int64_t)blockIdx.x : (int64_t)blockIdx.x * S::G + g) * o.per_unit;
+  const int sub = COOP ? g : 0;
+  const int T = (int)p.T;
+  const int iters = (T + GS - 1) / GS;  // steps per sample
+
+  const TX *const xp = static_cast<const TX *>(p.x);
+  const TY *const yp = static_cast<const TY *>(p.y);
+  const TX *const dop = static_cast<const TX *>(p.dout);
+  const TX *const dhp = static_cast<const TX *>(p.dh_up);
+  using VX = typename Raw8<TX>::vtype;
+  using VY = typename Raw8<TY>::vtype;
+
+  float wv[K][8], accW[K][8], gn[K][8], sn[K][8];
+  auto load_cond = [&](int s) {  // conditioning of the unit's sample s into (gn, sn)
+    const int64_t b = b0 + s;
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+      const int col = (k * S::R + rt) * 8;
+      if (s < o.per_unit && b < o.B && col < p.N) {
+        load8_dyn<true>(p.gate, p.dt_gate, b * p.ld_gate + col, 8, gn[k]);
+        load8_dyn<true>(p.scale, p.dt_scale, b * p.ld_scale + col, 8, sn[k]);
+      } else {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) gn[k][i] = sn[k][i] = 0.f;
+      }
+    }
+  };
+#pragma unroll
+  for (int k = 0; k < K; ++k) {
+    const int col = (k * S::R + rt) * 8;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) wv[k][i] = accW[k][i] = 0.f;
+    if (col < p.N) load8_dyn<true>(p.weight, p.dt_weight, col, 8, wv[k]);
+  }
+  load_cond(0);
+
+  struct Row {
+    BwdRow<TX, TY, K> rw;
+    float rs;
+  };
+  // row of step it of the unit's sample s
+  auto row_of = [&](int s, int it, int64_t &row) {
+    const int t = it * GS + sub;
+    const int64_t b = b0 + s;
+    row = b * p.T + t;
+    return s < o.per_unit && b < o.B && t < T;
+  };
+  auto load_row = [&](int s, int it, Row &r) {
+    int64_t row;
+    const bool in = row_of(s, it, row);
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+      const int col = (k * S::R + rt) * 8;
+      if (in && col < p.N) {
+        r.rw.x[k].v = stream_load_vec<VX, NTL>(xp + row * p.ld_x + col);
+        r.rw.y[k].v = stream_load_vec<VY, NTL>(yp + row * p.ld_y + col);
+        if (dop) r.rw.dout[k].v = stream_load_vec<VX, NTL>(dop + row * (int64_t)p.N + col);
+        else r.rw.dout[k].zero();
+        if (dhp) r.rw.dh[k].v = stream_load_vec<VX, NTL>(dhp + row * (int64_t)p.N + col);
+        else r.rw.dh[k].zero();
+      } else {
+        r.rw.x[k].zero(); r.rw.y[k].zero(); r.rw.dout[k].zero(); r.rw.dh[k].zero();
+      }
+    }
+    r.rs = in ? p.rstd[row] : 0.f;
+  };
+
+  float wo[K][8], gv[K][8], sc[K][8], accA[K][8], accS[K][8], accG[K][8];
+  auto begin_sample = [&](int s) {
+#pragma unroll
+    for (int k = 0; k < K; ++k)
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        gv[k][i] = gn[k][i];
+        sc[k][i] = 1.f + sn[k][i];
+        wo[k][i] = wv[k][i] * sc[k][i];
+        accA[k][i] = accS[k][i] = accG[k][i] = 0.f;
+      }
+    load_cond(s + 1);
+  };
+  auto work_row = [&](int s, int it, const Row &r) {
+    int64_t row;
+    const bool in = row_of(s, it, row);
+    float xh[K][8], dot = 0.f;
+#pragma unroll
+    for (int k = 0; k < K; ++k)
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        xh[k][i] = (r.rw.x[k][i] + gv[k][i] * r.rw.y[k][i]) * r.rs;
+        dot += (r.rw.dout[k][i] * wo[k][i]) * xh[k][i];
+      }
+    dot = row_sum<WPR>(dot, red, g, rt);
+    const float c = dot / (float)p.N;
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+      const int col = (k * S::R + rt) * 8;
+      if (in && col < p.N) {
+        float dh[8], dyv[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+          const float d = r.rw.dout[k][i];
+          dh[i] = r.rw.dh[k][i] + r.rs * (d * wo[k][i] - xh[k][i] * c);
+          dyv[i] = dh[i] * gv[k][i];
+          accA[k][i] += d * xh[k][i];
+          accS[k][i] += d;
+          accG[k][i] += dh[i] * r.rw.y[k][i];
+        }
+        store8_hint<TX, true, NT>(static_cast<TX *>(p.dx) + row * (int64_t)p.N + col, 8, dh);
+        store8_hint<TY, true, NT>(static_cast<TY *>(p.dy) + row * (int64_t)p.N + col, 8, dyv);
+      }
+    }
+  };
+  auto end_sample = [&](int s) {
+    if constexpr (COOP && S::G > 1) {
+      combine_groups_lds<K, S::G, S::R>(accA, comb, g, rt);
+      combine_groups_lds<K, S::G, S::R>(accS, comb, g, rt);
+      combine_groups_lds<K, S::G, S::R>(accG, comb, g, rt);
+    }
+    const int64_t b = b0 + s;
+    if (sub != 0 || b >= o.B) return;
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+      const int col = (k * S::R + rt) * 8;
+      if (col < p.N) {
+        float ds[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+          ds[i] = wv[k][i] * accA[k][i];
+          accW[k][i] += sc[k][i] * accA[k][i];
+        }
+        const int64_t off = b * p.N + col;
+        if (o.dscale) store8_dyn(o.dscale, p.dt_scale, off, ds);
+        if (o.dshift) store8_dyn(o.dshift, o.dt_shift, off, accS[k]);
+        if (o.dgate) store8_dyn(o.dgate, p.dt_gate, off, accG[k]);
+      }
+    }
+  };
+
+  // the flattened steps, two per turn: (s, it) is buffer A's, (s2, it2) B's
+  auto next = [&](int &s, int &it) {
+    if (++it == iters) {
+      it = 0;
+      ++s;
+    }
+  };
+  Row A, B;
+  int s = 0, it = 0;
+  load_row(0, 0, A);
+  while (s < o.per_unit) {
+    int s2 = s, it2 = it;
+    next(s2, it2);
+    load_row(s2, it2, B);
+    if (it == 0) begin_sample(s);
+    work_row(s, it, A);
+    if (it == iters - 1) end_sample(s);
+    if (s2 >= o.per_unit) break;
+    s = s2;
+    it = it2;
+    next(s, it);
+    load_row(s, it, A);
+    if (it2 == 0) begin_sample(s2);
+    work_row(s2, it2, B);
+    if (it2 == iters - 1) end_sample(s2);
+  }
+
+  // the block's dweight row: the groups' shares in group order (COOP: group 0
+  // holds it all)
+  if constexpr (!COOP && S::G > 1) combine_groups_lds<K, S::G, S::R>(accW, comb, g, rt);
+  if (g == 0) {
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+      const int col = (k * S::R + rt) * 8;
+      if (col < p.N) Chunk8<float>::store(o.wpart + (int64_t)blockIdx.x * p.N + col, accW[k]);
+    }
+  }
+}
+
+// ---------------------------------------------------------------------------
 // planning
 // ---------------------------------------------------------------------------
 struct Plan {
@@ -828,6 +1051,37 @@ inline Plan make_plan(int64_t M, int64_t N, int64_t T, const Knobs &kn = Knobs()
   return pl;
 }
 
+// The sample-walking backward (adaln_bwd_walk_kernel): units of consecutive
+// samples, per_unit of them each, dealt to `blocks` blocks.
+struct WalkPlan {
+  bool use, coop;
+  int per_unit;
+  unsigned blocks;
+};
+// It runs when the plan would give every sample a block of its own and more
+// than one round of them (B above the blocks aimed at); with fewer samples
+// the blocks of adaln_bwd_kernel are all resident and the reduction takes at
+// most 8 rounds.  A row group walks samples alone when that makes at least
+// kWalkGroupWaves wavefronts (8 per CU), or when the sample has fewer rows
+// than a block has groups; otherwise the block's groups share each sample.
+constexpr int kWalkGroupWaves = 2048;
+constexpr int kWalkMaxBlocks = 1024;  // also the dweight rows to be added
+inline WalkPlan make_walk_plan(const Plan &pl, int64_t N, int64_t T) {
+  WalkPlan w{};
+  w.use = pl.B > kBwdBlocksTarget && T <= INT32_MAX / 64 && N % 8 == 0 &&
+          (pl.bwd_k == 1 ? pl.bwd_wpr <= 8 : pl.bwd_wpr == 8);
+  if (!w.use) return w;
+  const int R = 64 * pl.bwd_wpr;
+  const int G = (R < kWalkMinBlock ? kWalkMinBlock : R) / R;
+  w.coop = G > 1 && T >= G && pl.B * pl.bwd_wpr < kWalkGroupWaves;
+  const int64_t per_block = w.coop ? 1 : G;  // units per block
+  int64_t pu = (pl.B + per_block * kWalkMaxBlocks - 1) / (per_block * kWalkMaxBlocks);
+  w.per_unit = (int)pu;
+  const int64_t units = (pl.B + pu - 1) / pu;
+  w.blocks = (unsigned)((units + per_block - 1) / per_block);
+  return w;
+}
+
 inline size_t workspace_bytes(const Plan &pl, int64_t N) {
   return (size_t)(pl.B * pl.J * 3 * N) * sizeof(float);
 }
@@ -905,6 +1159,16 @@ int launch_bwd_t(const BwdArgs &a, const Plan &pl, hipStream_t s) {
     adaln_bwd_kernel<TX, TY, K, WPR, VEC, kBwdNT, PF, 512, CL><<<grid, S::BLK, 0, s>>>(a);
   }
   return check_launch("nf_adaln_bwd");
+}
+
+template <typename TX, typename TY, int WPR, int K>
+int launch_walk_t(const BwdArgs &a, const WalkOut &o, const WalkPlan &w, hipStream_t s) {
+  constexpr int BLK = BwdShape<WPR, kWalkMinBlock>::BLK;
+  if (w.coop)
+    adaln_bwd_walk_kernel<TX, TY, K, WPR, true, kBwdNT, false><<<w.blocks, BLK, 0, s>>>(a, o);
+  else
+    adaln_bwd_walk_kernel<TX, TY, K, WPR, false, kBwdNT, false><<<w.blocks, BLK, 0, s>>>(a, o);
+  return check_launch("nf_adaln_bwd_full");
 }
 
 // (wavefronts per row, chunks per lane) pairs make_plan gives on the vector
@@ -986,6 +1250,18 @@ int fwd_v(const FwdArgs &a, const Plan &pl, bool vec, hipStream_t s) {
 template <typename TX, typename TY>
 int bwd_v(const BwdArgs &a, const Plan &pl, bool vec, hipStream_t s) {
   return vec ? bwd_w<TX, TY, true>(a, pl, s) : bwd_w<TX, TY, false>(a, pl, s);
+}
+
+template <typename TX, typename TY>
+int bwd_walk(const BwdArgs &a, const WalkOut &o, const Plan &pl, const WalkPlan &w,
+             hipStream_t s) {
+  if (pl.bwd_k == 2) return launch_walk_t<TX, TY, 8, 2>(a, o, w, s);
+  switch (pl.bwd_wpr) {
+    case 1: return launch_walk_t<TX, TY, 1, 1>(a, o, w, s);
+    case 2: return launch_walk_t<TX, TY, 2, 1>(a, o, w, s);
+    case 4: return launch_walk_t<TX, TY, 4, 1>(a, o, w, s);
+    default: return launch_walk_t<TX, TY, 8, 1>(a, o, w, s);
+  }
 }
 
 // supported (x, y) type pairs: equal types, or fp32 residual with a 16-bit

@@ -5,5 +5,7 @@ namespace nf {
 namespace adaln {
 template int fwd_v<float, float>(const FwdArgs &, const Plan &, bool, hipStream_t);
 template int bwd_v<float, float>(const BwdArgs &, const Plan &, bool, hipStream_t);
+template int bwd_walk<float, float>(const BwdArgs &, const WalkOut &, const Plan &,
+                                 const WalkPlan &, hipStream_t);
 }  // namespace adaln
 }  // namespace nf

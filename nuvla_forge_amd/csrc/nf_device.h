@@ -246,6 +246,16 @@ __device__ __forceinline__ void store_dyn(void *p, int dt, int64_t off,
     static_cast<f16 *>(p)[off] = static_cast<f16>(v);
 }
 
+// Runtime-typed chunk store, 16-byte aligned.
+__device__ __forceinline__ void store8_dyn(void *p, int dt, int64_t off, const float (&v)[8]) {
+  if (dt == NF_DTYPE_F32)
+    Chunk8<float>::store(static_cast<float *>(p) + off, v);
+  else if (dt == NF_DTYPE_BF16)
+    Chunk8<bf16>::store(static_cast<bf16 *>(p) + off, v);
+  else
+    Chunk8<f16>::store(static_cast<f16 *>(p) + off, v);
+}
+
 // ---------------------------------------------------------------------------
 // Wavefront reductions.  Steps inside a 16-lane DPP row use quad_perm and the
 // row mirrors (each pairs every lane with a partner in the other half of its

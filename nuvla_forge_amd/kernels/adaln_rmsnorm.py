@@ -120,26 +120,18 @@ class _FusedAdaLNResidualRMSNorm(torch.autograd.Function):
         ws_bytes = L.nf_adaln_bwd_workspace(m, n, t)
         ws = torch.empty(max(ws_bytes, 1), dtype=torch.uint8, device=dev)
         with device_of(x):
-            stream = _lib.stream_of(x)
             _lib.check(
-                L.nf_adaln_bwd(
+                L.nf_adaln_bwd_full(
                     _lib.ptr(dh_up), _lib.ptr(dout),
                     x.data_ptr(), x.stride(0), y.data_ptr(), y.stride(0),
                     gate.data_ptr(), gate.stride(0), weight.data_ptr(),
                     scale.data_ptr(), scale.stride(0), rstd.data_ptr(),
-                    dx.data_ptr(), dy.data_ptr(), ws.data_ptr(), ws_bytes, m, n, t,
-                    dc(x), dc(y), dc(gate), dc(weight), dc(scale), stream,
+                    dx.data_ptr(), dy.data_ptr(), _lib.ptr(dgate), _lib.ptr(dweight),
+                    _lib.ptr(dscale), _lib.ptr(dshift), ws.data_ptr(), ws_bytes, m, n, t,
+                    dc(x), dc(y), dc(gate), dc(weight), dc(scale), dc(ctx.shift_dtype),
+                    _lib.stream_of(x),
                 ),
-                "nf_adaln_bwd",
-            )
-            _lib.check(
-                L.nf_adaln_bwd_reduce(
-                    ws.data_ptr(), ws_bytes, weight.data_ptr(), scale.data_ptr(),
-                    scale.stride(0), _lib.ptr(dgate), _lib.ptr(dweight), _lib.ptr(dscale),
-                    _lib.ptr(dshift), m, n, t, dc(gate), dc(weight), dc(scale),
-                    dc(ctx.shift_dtype), stream,
-                ),
-                "nf_adaln_bwd_reduce",
+                "nf_adaln_bwd_full",
             )
         return (dx if need[0] else None, dy if need[1] else None,
                 dgate, dweight, dscale, dshift, None, None)

@@ -115,6 +115,39 @@ def test_adaln_wide_rows(cuda, dtype, b, t, n):
         assert torch.equal(again[k], grads[k]), f"d{k} differs between runs"
 
 
+@pytest.mark.parametrize("xd,yd,b,t,n", [
+    (torch.float32, torch.bfloat16, 257, 1, 8),      # one row a sample, one lane a row
+    (torch.float32, torch.bfloat16, 2300, 3, 384),   # a group per sample, groups past the last
+    (torch.bfloat16, torch.bfloat16, 4500, 2, 72),   # two samples a group, a ragged last unit
+    (torch.float32, torch.float32, 261, 5, 520),     # groups of two wavefronts share a sample
+    (torch.bfloat16, torch.bfloat16, 300, 33, 1024),  # a block per sample, odd rows
+    (torch.float16, torch.float16, 1030, 2, 1536),   # four wavefronts a row
+    (torch.bfloat16, torch.bfloat16, 1100, 1, 4096),  # two samples a block, eight wavefronts
+    (torch.bfloat16, torch.bfloat16, 258, 2, 8192),  # two chunks a lane
+])
+def test_adaln_backward_over_many_samples(cuda, xd, yd, b, t, n):
+    """More samples than the row kernel's blocks: the sample-walking backward,
+    against the oracle; a second run is bit-identical, and a run that wants
+    only some of the parameter gradients gives the same ones."""
+    note(f"adaln many samples {xd}/{yd} b={b} t={t} n={n}")
+    inp = _inputs(b, t, n, xd, cuda, cond_dtype=yd, y_dtype=yd)
+    dh, dout = _upstream(b * t, n, xd, cuda)
+    h, out, grads = _run(inp, t, dh, dout)
+    # per tensor: the tolerance of its own type
+    a = {k: np64(v) for k, v in inp.items()}
+    gw = on.adaln_backward(**a, t=t, dh_up=np64(dh), dout=np64(dout), eps=1e-6)
+    for k in NAMES:
+        assert on.rel_err(np64(grads[k]), gw[k]) <= TOL[grads[k].dtype], k
+    _, _, again = _run(inp, t, dh, dout)
+    for k in NAMES:
+        assert torch.equal(again[k], grads[k]), f"d{k} differs between runs"
+    leaves = {k: v.detach().requires_grad_(k in ("x", "shift", "weight")) for k, v in inp.items()}
+    outs = fused_adaln_residual_rmsnorm(**leaves, tokens_per_sample=t)
+    got = torch.autograd.grad(outs, [leaves[k] for k in ("x", "shift", "weight")], [dh, dout])
+    for k, v in zip(("x", "shift", "weight"), got):
+        assert torch.equal(v, grads[k]), f"d{k} alone differs"
+
+
 def test_cfg2_bf16_and_bitwise_deterministic_backward(cuda):
     note("adaln cfg2 bf16 [8,1024,1024] x10 backward")
     b, t, n = 8, 1024, 1024
