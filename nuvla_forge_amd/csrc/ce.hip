@@ -754,15 +754,17 @@ struct Split {
   int S;
   int64_t kslice;
 };
+// dcols: tile extent along D (C::BN, or 192: then a stage is 3/4 the work).
 template <class C>
-inline Split dh_split(int64_t crows, int64_t D, int64_t V, int64_t ldp, bool single) {
-  const int64_t tn = (D + C::BN - 1) / C::BN;
+inline Split dh_split(int64_t crows, int64_t D, int64_t V, int64_t ldp, bool single,
+                      int64_t dcols) {
+  const int64_t tn = (D + dcols - 1) / dcols;
   const double tw = (double)((V + C::BM - 1) / C::BM * tn);
   const double th = (double)((crows + C::BM - 1) / C::BM * tn);
   // the N-major dW product (single) issues 8 LDS reads per 8 MFMAs against
   // 6: ~12% longer stages measured at K = 2048 / 4096
   const double kw = (double)crows / C::BK * (single ? 1.12 : 1.0);
-  const double stage_s = 2e-6, hbm_bps = 5e12;
+  const double stage_s = 2e-6 * (double)dcols / C::BN, hbm_bps = 5e12;
   Split best{1, ldp};
   double best_t = -1.0;
   for (int S = 1; S <= 64; ++S) {
@@ -792,6 +794,8 @@ struct Plan {
   // N-major, so a chunk holds twice the rows of the two-layout form in the
   // same bytes, and the fp32 dW accumulator is kept transposed, [D, ldp]
   bool single;
+  // d192: the gradient products' tiles take 192 of the D extent, not 256
+  bool d192;
   // state (kept from nf_ce_fwd to nf_ce_bwd)
   size_t s_scal, s_pos, s_cfac, s_wt, s_hct, s_p, s_pt, s_dhc, s_dwacc, s_total;
   // forward scratch
@@ -799,6 +803,15 @@ struct Plan {
   // backward scratch
   size_t b_part, b_total;
 };
+
+// Row stride, in elements of `es` bytes, of a matrix whose rows are read in
+// 128-byte K slices: whole 128-byte lines once that pads a row by less than
+// 1.6%, so a slice is one line and not parts of two.  V 50001 and M 12289 at
+// D 384, forward + backward: 2.39 ms with padded rows, 2.61 with rows of whole
+// 16-byte vectors.
+inline int64_t line_stride(int64_t n, size_t es) {
+  return n < 4096 ? round_up(n, 8) : round_up(n, 128 / (int64_t)es);
+}
 
 template <typename TI>
 inline Plan make_plan(int64_t M, int64_t D, int64_t V, int64_t chunk_rows) {
@@ -835,14 +848,17 @@ inline Plan make_plan(int64_t M, int64_t D, int64_t V, int64_t chunk_rows) {
     P.crows = cr > mcap ? mcap : cr;
   }
   P.nch = (M + P.crows - 1) / P.crows;
-  P.ldp = round_up(V, 8);
+  P.ldp = line_stride(V, es);
   P.ldwt = P.ldp;
-  P.ldht = round_up(M, 8);
+  P.ldht = line_stride(M, es);
   P.wtm = C::WTM;
   P.vtiles = (int)((V + C::BM - 1) / C::BM);
   P.ntiles = P.vtiles * C::WM;
   P.ttiles = (int)(P.crows / C::BN);
-  P.split = dh_split<C>(P.crows, D, V, P.ldp, P.single);
+  // With E held once D is a tile extent of both gradient products (rows of
+  // dW^T, columns of dH); a 192 tile reads ~6% more operand per product.
+  P.d192 = P.single && round_up(D, 192) * 1.06 < round_up(D, 256);
+  P.split = dh_split<C>(P.crows, D, V, P.ldp, P.single, P.d192 ? 192 : C::BN);
   const size_t part = P.split.S > 1 ? (size_t)P.split.S * P.crows * D * sizeof(float) : 0;
   size_t o = 0;
   auto take = [&](size_t bytes) { const size_t at = o; o = align256(o + bytes); return at; };
@@ -902,17 +918,17 @@ struct StateView {
 // given.
 // reduce_dh = false leaves a split dH's fp32 slices in `part` for the
 // caller (the backward's scatter adds them).
-template <typename TI>
-int launch_grads(const Plan &L, const StateView<TI> &S, int64_t c, int64_t D, int64_t V,
+// C, CT: the tilings of the products with a K-contiguous and an N-major B.
+template <typename TI, class C, class CT>
+int launch_grads_tiled(const Plan &L, const StateView<TI> &S, int64_t c, int64_t D, int64_t V,
                  const float *dw_in, void *dw_out, int dt_w, const float *g, float *part,
                  hipStream_t s, bool final_dw, bool reduce_dh = true) {
-  using C = MainCfg<TI>;
   const int64_t j0 = c * L.crows;
   // single: dW^T (+)= Hct_c P_c, [D, V], with P read N-major; the fp32
   // accumulator holds dW^T [D, ldp] and the final product stores dW [V, D]
   // transposed (final_dw: dw_out is the caller's gradient).
-  auto jw = L.single ? make_job<C>(S.Hct + j0, L.ldht, S.P, L.ldp, dw_in, dw_out, dt_w, g,
-                                   final_dw ? D : L.ldp, D, V, L.crows)
+  auto jw = L.single ? make_job<CT>(S.Hct + j0, L.ldht, S.P, L.ldp, dw_in, dw_out, dt_w, g,
+                                    final_dw ? D : L.ldp, D, V, L.crows)
                      : make_job<C>(S.PT, L.crows, S.Hct + j0, L.ldht, dw_in, dw_out, dt_w, g,
                                    D, V, D, L.crows);
   if (L.single) {
@@ -936,9 +952,24 @@ int launch_grads(const Plan &L, const StateView<TI> &S, int64_t c, int64_t D, in
     jh.tiles *= L.split.S;
   }
   // the longest blocks go first (the dW job is never split)
-  return L.split.kslice > L.crows ? launch_gemm_store<C>(jh, jw, s, reduce_dh)
-                                  : launch_gemm_store<C>(jw, jh, s, reduce_dh);
+  return L.split.kslice > L.crows ? launch_gemm_store<C, CT>(jh, jw, s, reduce_dh)
+                                  : launch_gemm_store<C, CT>(jw, jh, s, reduce_dh);
 }
+
+template <typename TI>
+int launch_grads(const Plan &L, const StateView<TI> &S, int64_t c, int64_t D, int64_t V,
+                 const float *dw_in, void *dw_out, int dt_w, const float *g, float *part,
+                 hipStream_t s, bool final_dw, bool reduce_dh = true) {
+  using C = MainCfg<TI>;
+  if constexpr (sizeof(TI) == 2) {
+    if (L.d192)
+      return launch_grads_tiled<TI, Cols192Cfg, Rows192Cfg>(L, S, c, D, V, dw_in, dw_out, dt_w, g,
+                                                            part, s, final_dw, reduce_dh);
+  }
+  return launch_grads_tiled<TI, C, C>(L, S, c, D, V, dw_in, dw_out, dt_w, g, part, s, final_dw,
+                                      reduce_dh);
+}
+
 
 template <typename TI>
 int ce_fwd_run(const TI *H, const TI *W, const int64_t *targets, int64_t M, int64_t D,

@@ -167,7 +167,7 @@ constexpr bool ct_vec_tiling() {
   if constexpr (!C::DTL)
     return false;
   else
-    return C::WTN == 64 && C::WN * C::WTN == C::BN && C::BM == 256;
+    return C::WTN == 64 && C::WN * C::WTN == C::BN && C::BM % 64 == 0;
 }
 
 // One block's tile of job j: the K loop (B K-contiguous, or N-major when BT)
@@ -223,14 +223,14 @@ __device__ __forceinline__ void store_tile(const GemmJob<typename C::TI> &j, int
     // Transposed store through LDS (free after the K loop), so that global
     // stores are whole 16-byte vectors along m: in pass p the wavefronts of
     // column p (tile columns 64 p .. 64 p + 63) put their scaled accumulators
-    // into LDS as 64 rows n of 256 m (row pitch 256 elements + 16 bytes, so
+    // into LDS as 64 rows n of BM m (row pitch BM elements + 16 bytes, so
     // the 32 rows a write instruction touches start on different banks), then
     // every thread stores row vectors.  Needs M and ldc multiples of 8.
     const int es = dtype_bytes(cdt);
-    const int pitch = 256 * es + 16;
+    const int pitch = C::BM * es + 16;
     const int l = threadIdx.x & 63, w = threadIdx.x >> 6;
     const int wm = w / C::WN, wn = w % C::WN;
-    const int vpr = 256 * es / 16;  // 16-byte vectors per LDS row
+    const int vpr = C::BM * es / 16;  // 16-byte vectors per LDS row
 #pragma unroll 1
     for (int p = 0; p < C::WN; ++p) {
       if (wn == p) {
@@ -311,10 +311,13 @@ __device__ __forceinline__ void store_tile(const GemmJob<typename C::TI> &j, int
   }
 }
 
-template <class C, bool BUF, bool SB>
+// C tiles the jobs whose B is K-contiguous, CT those whose B is N-major (bt).
+template <class C, class CT, bool BUF, bool SB>
 __global__ NF_GEMM_BOUNDS(C) void gemm_store_kernel(GemmJob<typename C::TI> j0,
                                                     GemmJob<typename C::TI> j1) {
-  __shared__ __attribute__((aligned(16))) char smem[C::LDS_BYTES];
+  static_assert(C::NT == CT::NT, "one block size for both tilings");
+  __shared__ __attribute__((aligned(16)))
+  char smem[C::LDS_BYTES > CT::LDS_BYTES ? C::LDS_BYTES : CT::LDS_BYTES];
   // The job comes from the raw block index, so j0's blocks are dispatched
   // first and spread over all 8 XCDs (block b runs on XCD b % 8); the
   // XCD-grouped tile order applies within each job.  (Grouping the two jobs
@@ -337,7 +340,8 @@ __global__ NF_GEMM_BOUNDS(C) void gemm_store_kernel(GemmJob<typename C::TI> j0,
   const int tiles_n = j.tiles / j.ksplit / j.tiles_m;
   int tiles_m = j.tiles_m, tiles = j.tiles;
   if (j.dyn && j.dyn_rows) {
-    tiles_m = (int)((M + C::BM - 1) / C::BM);
+    const int bm = j.bt ? CT::BM : C::BM;
+    tiles_m = (int)((M + bm - 1) / bm);
     tiles = tiles_m * tiles_n * j.ksplit;
   }
   if (b >= tiles) return;
@@ -346,15 +350,13 @@ __global__ NF_GEMM_BOUNDS(C) void gemm_store_kernel(GemmJob<typename C::TI> j0,
   const int ks = t / per_split;  // K slice of this block
   int tm, tn;
   gemm::group_tile(t % per_split, tiles_m, tiles_n, gemm::kTileGroup, tm, tn);
-  const int64_t m0 = (int64_t)tm * C::BM;
-  const int64_t n0 = (int64_t)tn * C::BN;
-  if constexpr (kn_tiling<C>()) {
+  if constexpr (kn_tiling<CT>()) {
     if (j.bt) {
-      store_tile<C, BUF, SB, true>(j, M, K, ks, m0, n0, smem);
+      store_tile<CT, BUF, SB, true>(j, M, K, ks, (int64_t)tm * CT::BM, (int64_t)tn * CT::BN, smem);
       return;
     }
   }
-  store_tile<C, BUF, SB, false>(j, M, K, ks, m0, n0, smem);
+  store_tile<C, BUF, SB, false>(j, M, K, ks, (int64_t)tm * C::BM, (int64_t)tn * C::BN, smem);
 }
 
 // C[m, n] = scale * row_scale[m] * (Cin[m, n] + sum over s = 0 .. S-1 of
@@ -565,6 +567,10 @@ template <>
 struct MainCfgT<float> { using type = Cfg<float, 128, 128, 2, 2>; };
 template <typename TI>
 using MainCfg = typename MainCfgT<TI>::type;
+// 192 rows (B N-major) or columns (B K-contiguous) in the place of 256, for an
+// extent that 256 would pad much further (384: two of 192 against 512)
+using Rows192Cfg = gemm::DCfg<192, 256, 2, 4, 2, 64>;
+using Cols192Cfg = gemm::DCfg<256, 192, 4, 2, 2, 64>;
 
 inline int64_t round_up(int64_t x, int64_t m) { return (x + m - 1) / m * m; }
 inline size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
@@ -613,19 +619,20 @@ bool job_sb_ok(const GemmJob<TI> &j) {
 // Both jobs in one grid (j1 may be empty: tiles == 0), then the split-K
 // reductions of a split job (unless `reduce` is false: the caller then adds
 // the slices itself, as splitk_reduce_kernel would).
-template <class C>
+// Each job was made with the tiling it runs on: C, or CT with an N-major B.
+template <class C, class CT = C>
 int launch_gemm_store(const GemmJob<typename C::TI> &j0_in, const GemmJob<typename C::TI> &j1_in,
                       hipStream_t s, bool reduce = true) {
   GemmJob<typename C::TI> j0 = j0_in, j1 = j1_in;
   for (auto *jp : {&j0, &j1})  // the LDS-transposed store where it applies
-    jp->ct_vec = ct_vec_tiling<C>() && jp->ct && !jp->row_scale && jp->M % 8 == 0 &&
+    jp->ct_vec = (jp->bt ? ct_vec_tiling<CT>() : ct_vec_tiling<C>()) && jp->ct && !jp->row_scale && jp->M % 8 == 0 &&
                  jp->ldc % 8 == 0;
   const int64_t total = (int64_t)j0.tiles + j1.tiles;
   if (total == 0) return NF_OK;
   if (total > 0x7fffffffLL) return set_error(NF_ERR_ARG, "gemm: too many tiles");
   for (const auto *jp : {&j0, &j1}) {
     if (jp->tiles == 0) continue;
-    if (jp->bt && !kn_tiling<C>())
+    if (jp->bt && !kn_tiling<CT>())
       return set_error(NF_ERR_ARG, "gemm: an N-major B needs the 16-bit 256-column tiling");
     if (jp->ct && jp->ksplit > 1)
       return set_error(NF_ERR_ARG, "gemm: a transposed C cannot be split along K");
@@ -634,11 +641,11 @@ int launch_gemm_store(const GemmJob<typename C::TI> &j0_in, const GemmJob<typena
   const bool sb = job_sb_ok(j0) && job_sb_ok(j1);
   const bool buf = job_buf_ok(j0) && job_buf_ok(j1);
   if (buf && sb)
-    gemm_store_kernel<C, true, true><<<grid, C::NT, 0, s>>>(j0, j1);
+    gemm_store_kernel<C, CT, true, true><<<grid, C::NT, 0, s>>>(j0, j1);
   else if (buf)
-    gemm_store_kernel<C, true, false><<<grid, C::NT, 0, s>>>(j0, j1);
+    gemm_store_kernel<C, CT, true, false><<<grid, C::NT, 0, s>>>(j0, j1);
   else
-    gemm_store_kernel<C, false, false><<<grid, C::NT, 0, s>>>(j0, j1);
+    gemm_store_kernel<C, CT, false, false><<<grid, C::NT, 0, s>>>(j0, j1);
   if (int e = check_launch("gemm_store")) return e;
   if (!reduce) return NF_OK;
   for (const auto *jp : {&j0, &j1}) {
