@@ -102,6 +102,23 @@ int nf_gemm_swiglu_wgrad(const void *da, const void *db, int64_t ld_ab,
                          int64_t H, int dtype, void *workspace,
                          size_t workspace_bytes, void *stream);
 
+/* All three products of the gate/up projection's backward in one launch (and
+ * one for the split-K sums): dx = da W_gate + db W_up ([M, D], dt_dx),
+ * dw_gate = da^T x and dw_up = db^T x ([H, D], dt_dw), contiguous, each NULL
+ * where not wanted; fp32 accumulation over both terms of dx, one rounding to
+ * the output type, fixed orders.  Operands, limits and M == 0 as in
+ * nf_gemm_swiglu and nf_gemm_swiglu_wgrad; the operands are read as they lie.
+ * Workspace: nf_gemm_swiglu_bwd_workspace bytes (may be 0), 16-byte aligned;
+ * its want flags say which outputs are not NULL. */
+size_t nf_gemm_swiglu_bwd_workspace(int64_t M, int64_t D, int64_t H,
+                                    int want_dx, int want_dgate, int want_dup);
+int nf_gemm_swiglu_bwd(const void *da, const void *db, int64_t ld_ab,
+                       const void *x, int64_t ldx, const void *w_gate,
+                       int64_t ld_gate, const void *w_up, int64_t ld_up,
+                       void *dx, int dt_dx, void *dw_gate, void *dw_up,
+                       int dt_dw, int64_t M, int64_t D, int64_t H, int dtype,
+                       void *workspace, size_t workspace_bytes, void *stream);
+
 /* ------------------------------------------------------------------------
  * adaLN-Zero seam: gated residual add, RMSNorm, modulation.  Row m of the
  * [M, N] activations belongs to sample m / T (M = B * T).

@@ -508,6 +508,42 @@ __device__ __forceinline__ void read_kgroup_kn(const char *stage, int wm, int wn
   }
 }
 
+// Operands of one 16-wide k-group with A M-major ([K, M], unit-stride M; the
+// stage layout of an N-major B, DtlOperandKN over BM columns) and B N-major
+// (BKN) or K-contiguous.  MFMA tile i's slot differs from tile 0's in bits 2
+// and 3 only, which no other term of the address sets.
+template <class C, bool BKN>
+__device__ __forceinline__ void read_kgroup_km(const char *stage, int wm, int wn, int kg,
+                                               u32x4 (&a)[C::TM], u32x4 (&b)[C::TN]) {
+  typedef short v4s __attribute__((ext_vector_type(4)));
+  typedef __attribute__((address_space(3))) v4s *lds_v4s;
+  static_assert(C::BM == 256 && C::BN == 256 && C::WTM == 128 && C::WTN == 64, "M-major A tiling");
+  const int l = threadIdx.x & 63, j16 = l & 15;
+  const int r = 8 * (l >> 5) + (j16 >> 2);                 // k-row at kg = 0
+  const int c = 16 * ((l >> 4) & 1) + 4 * (j16 & 3);       // column within an MFMA tile
+  auto tr8 = [](const char *p) {
+    const v4s x = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s)p);
+    const v4s y = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s)(p + 4 * (2 * 256)));
+    return __builtin_bit_cast(u32x4, __builtin_shufflevector(x, y, 0, 1, 2, 3, 4, 5, 6, 7));
+  };
+  auto off = [&](int col) { return r * 512 + (((col >> 3) ^ kn_swz<C>(r)) << 4) + (col & 7) * 2; };
+  const int offa = off(wm * C::WTM + c);
+  const char *as = stage + kg * 16 * 512;
+#pragma unroll
+  for (int i = 0; i < C::TM; ++i) a[i] = tr8(as + (offa ^ (64 * i)));
+  if constexpr (BKN) {
+    const int offb = off(wn * C::WTN + c);
+#pragma unroll
+    for (int j = 0; j < C::TN; ++j) b[j] = tr8(as + C::BM * C::ROW + (offb ^ (64 * j)));
+  } else {
+    const int sw = dtl_slot<C>(l & 31, 2 * kg + (l >> 5)) * 16;
+    const char *bs = stage + (C::BM + wn * C::WTN + (l & 31)) * C::ROW + sw;
+#pragma unroll
+    for (int j = 0; j < C::TN; ++j)
+      b[j] = *reinterpret_cast<const u32x4 *>(bs + j * 32 * C::ROW);
+  }
+}
+
 // ---- 16x16x32 products on K-contiguous operands -------------------------------
 #ifndef NF_MFMA16
 #define NF_MFMA16 1
@@ -683,19 +719,20 @@ __device__ __forceinline__ void mainloop_dtl16(const DtlOperand<C, C::ACW> &opa,
     for (int j = 0; j < C::TN; ++j) acc_swap16(acc[i][j]);
 }
 
-// k-group operands for B operand type OpB
-template <class C, class OpB>
+// k-group operands for operand types OpA, OpB
+template <class C, class OpA, class OpB>
 __device__ __forceinline__ void read_kgroup_op(const char *stage, int wm, int wn, int kg,
                                                u32x4 (&a)[C::TM], u32x4 (&b)[C::TN]) {
-  if constexpr (OpB::kKRows)
+  if constexpr (OpA::kKRows)
+    read_kgroup_km<C, OpB::kKRows>(stage, wm, wn, kg, a, b);
+  else if constexpr (OpB::kKRows)
     read_kgroup_kn<C>(stage, wm, wn, kg, a, b);
   else
     read_kgroup_dtl<C>(stage, wm, wn, kg, a, b);
 }
 
-template <class C, bool BUF, bool ZERO = false, class OpB>
-__device__ __forceinline__ void mainloop_dtl_ops(const DtlOperand<C, C::ACW> &opa,
-                                                 const OpB &opb, int64_t K,
+template <class C, bool BUF, bool ZERO = false, class OpA, class OpB>
+__device__ __forceinline__ void mainloop_dtl_ops(const OpA &opa, const OpB &opb, int64_t K,
                                                  char *smem, floatx16 (&acc)[C::TM][C::TN]);
 
 template <class C, bool BUF, bool ZERO>
@@ -746,18 +783,17 @@ __device__ __forceinline__ void mainloop_kn(const bf16 *A, int64_t lda, const bf
 
 // The K loop over operands the caller has set up (a kernel may point each
 // wavefront's share of a tile at a different matrix).  acc is not cleared.
-// OpB: DtlOperand (B K-contiguous) or DtlOperandKN (B N-major).  ZERO: acc
-// holds zeros on entry.
-template <class C, bool BUF, bool ZERO, class OpB>
-__device__ __forceinline__ void mainloop_dtl_ops(const DtlOperand<C, C::ACW> &opa,
-                                                 const OpB &opb, int64_t K,
+// OpA, OpB: DtlOperand (K-contiguous) or DtlOperandKN (A M-major, B N-major).
+// ZERO: acc holds zeros on entry.
+template <class C, bool BUF, bool ZERO, class OpA, class OpB>
+__device__ __forceinline__ void mainloop_dtl_ops(const OpA &opa, const OpB &opb, int64_t K,
                                                  char *smem, floatx16 (&acc)[C::TM][C::TN]) {
-  if constexpr (!OpB::kKRows && C::BK == 64 && kMfma16) {
+  if constexpr (!OpA::kKRows && !OpB::kKRows && C::BK == 64 && kMfma16) {
     mainloop_dtl16<C, BUF, ZERO>(opa, opb, K, smem, acc);
     return;
   }
-  // LDS read instructions per k-group: an N-major B takes two per MFMA tile
-  constexpr int kReadsB = C::TM + (OpB::kKRows ? 2 : 1) * C::TN;
+  // LDS read instructions per k-group: an M- / N-major operand takes two per MFMA tile
+  constexpr int kReadsB = (OpA::kKRows ? 2 : 1) * C::TM + (OpB::kKRows ? 2 : 1) * C::TN;
   const int w = threadIdx.x >> 6;
   const int wave = __builtin_amdgcn_readfirstlane(w);
   const int wm = w / C::WN, wn = w % C::WN;
@@ -782,7 +818,7 @@ __device__ __forceinline__ void mainloop_dtl_ops(const DtlOperand<C, C::ACW> &op
       }
     if (nk > 0) {
       wait_stage<C>(nk - 1 < C::STAGES - 1 ? (int)(nk - 1) : C::STAGES - 1);
-      read_kgroup_op<C, OpB>(smem, wm, wn, 0, a0, b0);
+      read_kgroup_op<C, OpA, OpB>(smem, wm, wn, 0, a0, b0);
     }
     int cur = 0;  // buffer of stage kt
     static_assert(C::KG % 2 == 0, "k-groups alternate register sets in pairs");
@@ -790,11 +826,11 @@ __device__ __forceinline__ void mainloop_dtl_ops(const DtlOperand<C, C::ACW> &op
       const char *st = smem + cur * C::STAGE;
 #pragma unroll
       for (int kg = 0; kg + 1 < C::KG; kg += 2) {
-        read_kgroup_op<C, OpB>(st, wm, wn, kg + 1, a1, b1);
+        read_kgroup_op<C, OpA, OpB>(st, wm, wn, kg + 1, a1, b1);
         mfma_block<C>(a0, b0, acc);
         interleave_hint<C, kReadsB>();
         if (kg + 2 < C::KG) {
-          read_kgroup_op<C, OpB>(st, wm, wn, kg + 2, a0, b0);
+          read_kgroup_op<C, OpA, OpB>(st, wm, wn, kg + 2, a0, b0);
           mfma_block<C>(a1, b1, acc);
           interleave_hint<C, kReadsB>();
         }
@@ -815,7 +851,7 @@ __device__ __forceinline__ void mainloop_dtl_ops(const DtlOperand<C, C::ACW> &op
           opb.issue((kt + C::STAGES) * C::BK, re + C::BM * C::ROW, wave);
         }
         cur = cur + 1 == C::STAGES ? 0 : cur + 1;
-        read_kgroup_op<C, OpB>(smem + cur * C::STAGE, wm, wn, 0, a0, b0);
+        read_kgroup_op<C, OpA, OpB>(smem + cur * C::STAGE, wm, wn, 0, a0, b0);
       }
     }
   } else {
@@ -825,8 +861,8 @@ __device__ __forceinline__ void mainloop_dtl_ops(const DtlOperand<C, C::ACW> &op
       __syncthreads();
 #pragma unroll
       for (int kg = 0; kg < C::KG; kg += 2) {
-        read_kgroup_op<C, OpB>(smem, wm, wn, kg, a0, b0);
-        read_kgroup_op<C, OpB>(smem, wm, wn, kg + 1, a1, b1);
+        read_kgroup_op<C, OpA, OpB>(smem, wm, wn, kg, a0, b0);
+        read_kgroup_op<C, OpA, OpB>(smem, wm, wn, kg + 1, a1, b1);
         mfma_block<C>(a0, b0, acc);
         mfma_block<C>(a1, b1, acc);
       }

@@ -111,25 +111,24 @@ class _FusedGateUpSwiGLU(torch.autograd.Function):
                 "nf_swiglu_bwd",
             )
         need = ctx.needs_input_grad
-        dx = torch.addmm(torch.mm(da, w_gate), db, w_up) if need[0] else None
-        dwg = dwu = None
-        if need[1] or need[2]:
-            m, d = x.shape
-            h = a.shape[1]
-            dwg = torch.empty((h, d), dtype=torch.bfloat16, device=x.device)
-            dwu = torch.empty_like(dwg)
-            with device_of(x):
-                nbytes = L.nf_gemm_swiglu_wgrad_workspace(m, d, h)
-                ws = torch.empty(max(nbytes, 1), dtype=torch.uint8, device=x.device)
-                _lib.check(
-                    L.nf_gemm_swiglu_wgrad(da.data_ptr(), db.data_ptr(), da.stride(0),
-                                           x.data_ptr(), x.stride(0), dwg.data_ptr(),
-                                           dwu.data_ptr(), dwg.stride(0), m, d, h,
-                                           _lib.dtype_code(torch.bfloat16), ws.data_ptr(),
-                                           nbytes, _lib.stream_of(x)),
-                    "nf_gemm_swiglu_wgrad",
-                )
-        return dx, dwg if need[1] else None, dwu if need[2] else None
+        m, d = x.shape
+        h = a.shape[1]
+        dx = torch.empty((m, d), dtype=torch.bfloat16, device=x.device) if need[0] else None
+        dwg = torch.empty((h, d), dtype=torch.bfloat16, device=x.device) if need[1] else None
+        dwu = torch.empty((h, d), dtype=torch.bfloat16, device=x.device) if need[2] else None
+        code = _lib.dtype_code(torch.bfloat16)
+        with device_of(x):
+            nbytes = L.nf_gemm_swiglu_bwd_workspace(m, d, h, need[0], need[1], need[2])
+            ws = torch.empty(max(nbytes, 1), dtype=torch.uint8, device=x.device)
+            _lib.check(
+                L.nf_gemm_swiglu_bwd(da.data_ptr(), db.data_ptr(), da.stride(0), x.data_ptr(),
+                                     x.stride(0), w_gate.data_ptr(), w_gate.stride(0),
+                                     w_up.data_ptr(), w_up.stride(0), _lib.ptr(dx), code,
+                                     _lib.ptr(dwg), _lib.ptr(dwu), code, m, d, h, code,
+                                     ws.data_ptr(), nbytes, _lib.stream_of(x)),
+                "nf_gemm_swiglu_bwd",
+            )
+        return dx, dwg, dwu
 
 
 def _gate_up_eager(x, w_gate, w_up):
