@@ -91,6 +91,7 @@ SIGNATURES = {
 
 _lib: ctypes.CDLL | None = None
 _load_error: str | None = None
+_native = None
 
 
 def _open() -> ctypes.CDLL:
@@ -120,6 +121,21 @@ def lib() -> ctypes.CDLL:
             _load_error = str(e)
             raise RuntimeError(f"nuvla_forge_amd HIP library unavailable: {e}") from e
     return _lib
+
+
+def native():
+    """The extension module with the ops' C++ host side; raises RuntimeError if
+    it cannot be loaded."""
+    global _native
+    if _native is None:
+        lib()  # the product library first: its version is checked
+        try:
+            from . import _native as mod
+        except ImportError as e:
+            raise RuntimeError("nuvla_forge_amd/_native.so is not built or does not load; run "
+                               f"`python -m nuvla_forge_amd.build`: {e}") from e
+        _native = mod
+    return _native
 
 
 def available() -> bool:

@@ -6,7 +6,9 @@ compiled to an object in ``_build/`` (in parallel), then linked into
 The measurement aids and the GEMM test hook (``csrc/measure/*.hip``,
 include/nuvla_forge_measure.h) go into ``nuvla_forge_amd/libnf_measure.so``,
 which links the product library for its error reporting; only the benchmark
-and the tests load it.  Both link ``libamdhip64.so.7`` by soname, so inside a
+and the tests load it.  ``csrc/host/native_ops.cpp``, the ops' host side in C++ on torch's
+C++ API, becomes the extension module ``nuvla_forge_amd/_native.so``, which
+links the product library too.  All link ``libamdhip64.so.7`` by soname, so inside a
 process that imported torch first they bind to the HIP runtime torch already
 loaded.  Last, ``tests/c/abi_smoke`` (a C program using the product library
 through its C ABI alone) is compiled with gcc.
@@ -26,6 +28,7 @@ CSRC = PKG / "csrc"
 BUILD = PKG.parent / "_build"
 LIB = PKG / "libnf_hip.so"
 MEASURE_LIB = PKG / "libnf_measure.so"
+NATIVE = PKG / "_native.so"
 INCLUDE = PKG.parent / "include"
 
 ARCH = "gfx950"
@@ -83,20 +86,62 @@ def _link(objs: list[Path], out: Path, extra: list[str], verbose: bool) -> None:
     os.replace(tmp, out)
 
 
+def _torch_flags() -> tuple[list[str], list[str]]:
+    """g++ compile and link flags for a Python extension on torch's C++ API."""
+    import sysconfig
+
+    import torch
+
+    root = Path(torch.__file__).resolve().parent
+    rocm = Path(os.environ.get("ROCM_PATH", "/opt/rocm"))
+    inc = [root / "include", root / "include/torch/csrc/api/include", rocm / "include"]
+    cflags = ["-D__HIP_PLATFORM_AMD__", "-DUSE_ROCM",
+              f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+              *(f"-isystem{p}" for p in inc), f"-I{sysconfig.get_paths()['include']}"]
+    libs = [f"-L{root / 'lib'}", "-ltorch_python", "-ltorch", "-ltorch_cpu", "-lc10", "-lc10_hip"]
+    return cflags, libs
+
+
+def _compile_native(verbose: bool) -> Path:
+    src, obj = CSRC / "host" / "native_ops.cpp", BUILD / "native_ops.o"
+    cmd = [os.environ.get("CXX", "g++"), "-std=c++17", "-O2", "-fPIC", "-Wall", *_torch_flags()[0],
+           f"-I{INCLUDE}", "-c", str(src), "-o", str(obj)]
+    if verbose:
+        print(" ".join(cmd), flush=True)
+    res = subprocess.run(cmd, capture_output=True, text=True)
+    if res.returncode != 0:
+        raise RuntimeError(f"g++ failed on {src.name}:\n{res.stdout}{res.stderr}")
+    return obj
+
+
+def _link_native(obj: Path, verbose: bool) -> None:
+    tmp = NATIVE.with_suffix(".so.tmp")
+    cmd = [os.environ.get("CXX", "g++"), "-shared", "-o", str(tmp), str(obj), *_torch_flags()[1],
+           f"-L{PKG}", "-lnf_hip", "-Wl,-rpath,$ORIGIN"]
+    if verbose:
+        print(" ".join(cmd), flush=True)
+    res = subprocess.run(cmd, capture_output=True, text=True)
+    if res.returncode != 0:
+        raise RuntimeError(f"link of {NATIVE.name} failed:\n{res.stdout}{res.stderr}")
+    os.replace(tmp, NATIVE)
+
+
 def build(verbose: bool = False, jobs: int | None = None) -> Path:
     """Compile every csrc/*.hip and csrc/measure/*.hip for gfx950 and link
-    libnf_hip.so and libnf_measure.so.  Always rebuilds."""
+    libnf_hip.so, libnf_measure.so and _native.so.  Always rebuilds."""
     BUILD.mkdir(exist_ok=True)
     sources = sorted(CSRC.glob("*.hip"))
     measure = sorted((CSRC / "measure").glob("*.hip"))
     if not sources:
         raise RuntimeError(f"no sources under {CSRC}")
-    jobs = jobs or min(len(sources) + len(measure), max(1, (os.cpu_count() or 2)))
+    jobs = jobs or min(len(sources) + len(measure) + 1, max(1, (os.cpu_count() or 2)))
     with cf.ThreadPoolExecutor(max_workers=jobs) as ex:
+        native = ex.submit(_compile_native, verbose)
         objs = list(ex.map(lambda s: _compile(s, verbose), sources + measure))
     _link(objs[:len(sources)], LIB, ["-Wl,-soname,libnf_hip.so"], verbose)
     _link(objs[len(sources):], MEASURE_LIB,
           [f"-L{PKG}", "-lnf_hip", "-Wl,-rpath,$ORIGIN"], verbose)
+    _link_native(native.result(), verbose)
     build_c_smoke(verbose)
     return LIB
 

@@ -160,4 +160,8 @@ def fused_adaln_residual_rmsnorm(
     if x.shape[-1] > MAX_N or not use_fused(x, "fused_adaln_residual_rmsnorm",
                                              force_reference):
         return adaln_residual_rmsnorm_ref(x, y, gate, weight, scale, shift, tokens_per_sample, eps)
+    # the plain call runs in C++; any other (None) takes the Function above
+    pair = _lib.native().seam(x, y, gate, weight, scale, shift, tokens_per_sample, eps)
+    if pair is not None:
+        return pair
     return _FusedAdaLNResidualRMSNorm.apply(x, y, gate, weight, scale, shift, tokens_per_sample, eps)

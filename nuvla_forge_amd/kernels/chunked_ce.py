@@ -257,5 +257,11 @@ def chunked_cross_entropy(
 
     Host tensors run the reference's eager row-chunk loop, as in the reference.
     """
+    if not VALIDATE_TARGETS and use_fused(hidden, "chunked_cross_entropy", force_reference):
+        # the plain call runs in C++; any other (None) takes the Function above
+        loss = _lib.native().ce(hidden, lm_weight, targets, chunk_size, ignore_index,
+                                _lib.dtype_code(_compute_dtype(hidden, lm_weight)))
+        if loss is not None:
+            return loss
     return _ChunkedCrossEntropy.apply(hidden, lm_weight, targets, chunk_size, ignore_index,
                                       force_reference)

@@ -70,16 +70,19 @@ class _FusedSwiGLU(torch.autograd.Function):
 class _FusedGateUpSwiGLU(torch.autograd.Function):
     """act = silu(x W_gate^T) * (x W_up^T) with the SwiGLU in the GEMM epilogue.
 
-    forward: one ``nf_gemm_swiglu`` launch writes act and the bf16 a, b the
-    backward needs.  backward: ``nf_swiglu_bwd`` forms da, db from a, b and
-    dact (sigmoid recomputed); ``nf_gemm_swiglu_wgrad`` computes dW_gate =
-    da^T x and dW_up = db^T x in one split-K launch (a token sum added in a
-    fixed order); dx = da W_gate + db W_up runs as library GEMMs.
+    forward: the inputs in bf16 (cast where they are not), then one
+    ``nf_gemm_swiglu`` launch writes act and the bf16 a, b the backward needs.
+    backward: ``nf_swiglu_bwd`` forms da, db from a, b and dact (sigmoid
+    recomputed); ``nf_gemm_swiglu_bwd`` computes dx = da W_gate + db W_up,
+    dW_gate = da^T x and dW_up = db^T x in one launch, each written once in
+    its input's type (sums over K splits added in a fixed order).
     """
 
     @staticmethod
     def forward(ctx, x, w_gate, w_up):
         check_devices("fused_gate_up_swiglu", "x", dict(x=x, w_gate=w_gate, w_up=w_up))
+        ctx.dtypes = (x.dtype, w_gate.dtype, w_up.dtype)
+        x, w_gate, w_up = _rows_bf16(x), _rows_bf16(w_gate), _rows_bf16(w_up)
         m, d = x.shape
         h = w_gate.shape[0]
         a = torch.empty((m, h), dtype=torch.bfloat16, device=x.device)
@@ -113,22 +116,25 @@ class _FusedGateUpSwiGLU(torch.autograd.Function):
         need = ctx.needs_input_grad
         m, d = x.shape
         h = a.shape[1]
-        dx = torch.empty((m, d), dtype=torch.bfloat16, device=x.device) if need[0] else None
-        dwg = torch.empty((h, d), dtype=torch.bfloat16, device=x.device) if need[1] else None
-        dwu = torch.empty((h, d), dtype=torch.bfloat16, device=x.device) if need[2] else None
-        code = _lib.dtype_code(torch.bfloat16)
+        tx, tg, tu = ctx.dtypes
+        dx = torch.empty((m, d), dtype=tx, device=x.device) if need[0] else None
+        # both weight gradients leave the kernel in one type
+        dwg = torch.empty((h, d), dtype=tg, device=x.device) if need[1] else None
+        dwu = torch.empty((h, d), dtype=tg, device=x.device) if need[2] else None
         with device_of(x):
             nbytes = L.nf_gemm_swiglu_bwd_workspace(m, d, h, need[0], need[1], need[2])
             ws = torch.empty(max(nbytes, 1), dtype=torch.uint8, device=x.device)
             _lib.check(
-                L.nf_gemm_swiglu_bwd(da.data_ptr(), db.data_ptr(), da.stride(0), x.data_ptr(),
+                L.nf_gemm_swiglu_bwd(da.data_ptr(), db.data_ptr(), h, x.data_ptr(),
                                      x.stride(0), w_gate.data_ptr(), w_gate.stride(0),
-                                     w_up.data_ptr(), w_up.stride(0), _lib.ptr(dx), code,
-                                     _lib.ptr(dwg), _lib.ptr(dwu), code, m, d, h, code,
-                                     ws.data_ptr(), nbytes, _lib.stream_of(x)),
+                                     w_up.data_ptr(), w_up.stride(0), _lib.ptr(dx),
+                                     _lib.dtype_code(tx), _lib.ptr(dwg), _lib.ptr(dwu),
+                                     _lib.dtype_code(tg), m, d, h,
+                                     _lib.dtype_code(torch.bfloat16), ws.data_ptr(), nbytes,
+                                     _lib.stream_of(x)),
                 "nf_gemm_swiglu_bwd",
             )
-        return dx, dwg, dwu
+        return dx, dwg, dwu if dwu is None else dwu.to(tu)
 
 
 def _gate_up_eager(x, w_gate, w_up):
@@ -164,14 +170,16 @@ def fused_gate_up_swiglu(x: torch.Tensor, w_gate: torch.Tensor, w_up: torch.Tens
         return fused_swiglu(F.linear(x, w_gate), F.linear(x, w_up))
     lead = x.shape[:-1]
     x2 = x.reshape(-1, x.shape[-1])
-    with torch.autocast(x.device.type, enabled=False):
-        act = _FusedGateUpSwiGLU.apply(
-            _rows_bf16(x2), _rows_bf16(w_gate), _rows_bf16(w_up))
+    # the plain call runs in C++; any other (None) takes the Function above
+    act = _lib.native().gate_up(x2, w_gate, w_up)
+    if act is None:
+        with torch.autocast(x.device.type, enabled=False):
+            act = _FusedGateUpSwiGLU.apply(x2, w_gate, w_up)
     return act.reshape(*lead, w_gate.shape[0])
 
 
 def _rows_bf16(t: torch.Tensor) -> torch.Tensor:
-    """bf16 with unit-stride rows (a differentiable cast / copy only when needed)."""
+    """bf16 with unit-stride rows (a cast / copy only when needed)."""
     t = t.to(torch.bfloat16)
     return t if t.stride(-1) == 1 else t.contiguous()
 
@@ -188,4 +196,6 @@ def fused_swiglu(a: torch.Tensor, b: torch.Tensor, force_reference: bool = False
     """
     if not use_fused(a, "fused_swiglu", force_reference):
         return swiglu_ref(a, b)
-    return _FusedSwiGLU.apply(a, b)
+    # the plain call runs in C++; any other (None) takes the Function above
+    out = _lib.native().swiglu(a, b)
+    return out if out is not None else _FusedSwiGLU.apply(a, b)

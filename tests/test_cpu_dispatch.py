@@ -137,3 +137,19 @@ def test_chunked_ce_on_host_tensors_all_ignored():
     loss, dh, dw = _ce_run(hid, w, tgt, 4)
     assert torch.isfinite(loss) and float(loss.detach()) == 0.0
     assert torch.all(dh == 0) and torch.all(dw == 0)
+
+
+def test_native_route_leaves_host_and_meta_tensors_alone():
+    """The C++ host side answers None to tensors that are not the device's
+    and to arguments that are no tensors; the general path then decides."""
+    from nuvla_forge_amd import _lib
+
+    n = _lib.native()
+    a, i = torch.zeros(4, 8), torch.zeros(4, dtype=torch.int64)
+    for t in (a, a.to("meta")):
+        assert n.swiglu(t, t) is None
+        assert n.gate_up(t, t, t) is None
+        assert n.seam(t, t, t, t[0], t, t, 1, 1e-6) is None
+        assert n.ce(t, t, i, 16, -100, 1) is None
+    assert n.swiglu(a, None) is None and n.swiglu(a) is None
+    assert n.seam(a, a, a, a[0], a, a, 1, "eps") is None
