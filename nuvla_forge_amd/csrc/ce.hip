@@ -300,7 +300,8 @@ __global__ NF_GEMM_BOUNDS(C) void ce_logits_kernel(
     // E = exp(S - mref) relative to the row's reference (rows past V are -inf
     // and give 0; S - mref is exact where S is near mref, so the target's own
     // entry is exactly 1).  The tile's statistics
-    // follow from its sum: s = sum exp(S - mx) = exp(mref - mx) * sum E.  A
+    // follow from its sum: s = sum exp(S - mx) = sum E / exp(mx - mref), the
+    // divisor being the largest entry as formed (a lone entry gives 1).  A
     // tile more than kStatsGap below mref keeps s = 1: its share of the row
     // total, below exp(-kStatsGap) of the row maximum's, is under fp32
     // resolution.  Where the maximum lies more than kBaseGap above mref (a
@@ -322,7 +323,7 @@ __global__ NF_GEMM_BOUNDS(C) void ce_logits_kernel(
     se += __shfl_xor(se, 32);
     const float s = mx == -INFINITY ? 0.f
                     : own           ? -se
-                    : (mr - mx > kStatsGap ? 1.f : se * exp_f32(mr - mx));
+                    : (mr - mx > kStatsGap ? 1.f : se / exp_f32(mx - mr));
     if (half == 0 && tok < cnt) stats[(int64_t)stile * crows + tok] = make_float2(mx, s);
 
 #pragma unroll
@@ -342,20 +343,24 @@ __global__ NF_GEMM_BOUNDS(C) void ce_logits_kernel(
           // straight from the accumulators: E row-major and E^T (zero past
           // the chunk's rows, up to the K padding of the dW product)
           const int64_t c = crow0 + o;
+          if constexpr (ES == 2) {
 #pragma unroll
-          for (int q = 0; q < 4; ++q) {
-            const TI e = tok < cnt ? ev[q] : static_cast<TI>(0.f);
-            if constexpr (ES == 2) {
+            for (int q = 0; q < 4; ++q) {
+              const TI e = tok < cnt ? ev[q] : static_cast<TI>(0.f);
               uint16_t bits;
               __builtin_memcpy(&bits, &e, 2);
               eout.st16((tok * ldp + c + q) * ES, tok < cnt && c + q < ldp, bits);
               etout.st16(((c + q) * ldet + tok) * ES, c + q < V && tok < cnt8, bits);
-            } else {
-              eout.st32((tok * ldp + c + q) * ES, tok < cnt && c + q < ldp,
-                        static_cast<float>(e));
-              etout.st32(((c + q) * ldet + tok) * ES, c + q < V && tok < cnt8,
-                         static_cast<float>(e));
             }
+          } else {
+            // c and ldp are multiples of 4: the four entries are one vector
+            u32x4 pk;
+            __builtin_memcpy(&pk, ev, 16);
+            eout.st128((tok * ldp + c) * ES, tok < cnt && c < ldp, pk);
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+              etout.st32(((c + q) * ldet + tok) * ES, c + q < V && tok < cnt8,
+                         tok < cnt ? static_cast<float>(ev[q]) : 0.f);
           }
         }
       }

@@ -5,18 +5,13 @@
 //    k of row (l % 32), k-half (l / 32)) or, on the direct-to-LDS path with B
 //    K-contiguous, four v_mfma_f32_16x16x32_bf16 per 32x32 tile brought to
 //    the same accumulator layout (mainloop_dtl16).
-//  * f32 inputs use v_mfma_f32_32x32x2_f32: lane l supplies one k of row
-//    (l % 32); four MFMAs consume a 16-byte k-slab per lane half, the half
-//    h = l / 32 covering k = 4h .. 4h+3 of each 8-wide group (the sum over k
-//    is order-free, so this permutation of k between the MFMAs is exact).
+//  * f32 inputs are split into three bf16 parts and multiplied as six bf16
+//    products (SplitCfg, mainloop_split), more precise than the fp32 MFMAs at
+//    over twice their rate.
 //  * Accumulator (32x32, 16 fp32 per lane): register r of lane l holds
 //    row 8 * (r / 4) + 4 * (l / 32) + (r % 4), column l % 32.
 //
-// Two stagings of the operand tiles in LDS:
-//  * Cfg (bf16 and f32): a K-stage is 128 bytes of every tile row (64 bf16 /
-//    32 f32), loaded into registers and written to LDS with a 144-byte row
-//    pitch, which makes both the 16-byte row writes and the 16-byte MFMA
-//    operand reads (eight lanes, eight distinct rows) bank-conflict free.
+// Staging of the bf16 operand tiles in LDS:
 //  * DCfg (bf16): a K-stage is BK = 32 or 64 k of every tile row (64 or 128
 //    bytes), copied global -> LDS by the buffer unit (buffer_load_dwordx4 ...
 //    lds) with no register staging.  One such load writes 1 KB contiguously
@@ -40,32 +35,6 @@ namespace gemm {
 typedef float floatx16 __attribute__((ext_vector_type(16)));
 typedef float floatx4 __attribute__((ext_vector_type(4)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-
-template <typename TI_, int BM_, int BN_, int WM_, int WN_>
-struct Cfg {
-  using TI = TI_;
-  static constexpr int BM = BM_, BN = BN_, WM = WM_, WN = WN_;
-  static constexpr int NT = WM * WN * 64;        // threads per block
-  static constexpr int WTM = BM / WM;            // wave tile rows
-  static constexpr int WTN = BN / WN;            // wave tile cols
-  static constexpr int TM = WTM / 32;            // 32x32 MFMA tiles per wave (M)
-  static constexpr int TN = WTN / 32;            // 32x32 MFMA tiles per wave (N)
-  static constexpr int VE = 16 / sizeof(TI);     // elements per 16-byte vector
-  static constexpr int BK = 128 / sizeof(TI);    // k per stage
-  static constexpr int KV = 8;                   // 16-byte vectors per row per stage
-  static constexpr int PITCH = 144;              // LDS row pitch, bytes
-  static constexpr int STAGE = (BM + BN) * PITCH;
-  static constexpr int LDS_BYTES = 2 * STAGE;
-  static constexpr int AV = BM * KV / NT;        // A vectors per thread per stage
-  static constexpr int BV = BN * KV / NT;        // B vectors per thread per stage
-  // K-stages of global loads in flight ahead of the MFMAs (register sets):
-  // 2 for small wave tiles, whose short compute stage hides little latency,
-  // 1 where a second set would not fit beside the accumulators.
-  static constexpr int PF = (NT <= 256 && TM * TN <= 4) ? 2 : 1;
-  static constexpr bool DTL = false;
-  static_assert(BM % (WM * 32) == 0 && BN % (WN * 32) == 0, "tile/wave mismatch");
-  static_assert((BM * KV) % NT == 0 && (BN * KV) % NT == 0, "loader mismatch");
-};
 
 // Direct-to-LDS bf16 configuration (see the file comment): BK k per stage
 // (32 or 64: LDS rows of 64 or 128 bytes), STAGES stage buffers.
@@ -120,74 +89,6 @@ __device__ __forceinline__ u32x4 load_vec(const TI *base, int64_t ld,
   return r;
 }
 
-// Operand source for the K loop.  BUF (the fast path): a buffer resource
-// over the whole operand, each thread's 16-byte vectors addressed by one
-// 32-bit base offset plus uniform strides; a vector whose row is past the
-// matrix or whose k is past K gets an out-of-range offset, which the buffer
-// unit turns into zeros (no branches, no 64-bit address math).  Requires
-// K % VE == 0, 16-byte aligned rows and an operand under 2 GiB.
-// !BUF: plain pointer loads with per-element masking (any K, any alignment).
-template <class C, bool BUF>
-struct Operand {
-  using TI = typename C::TI;
-  const TI *base;
-  int64_t ld, rows, K, r0;
-  __amdgpu_buffer_rsrc_t rsrc;
-  uint32_t off0;       // byte offset of this thread's first vector at k = 0
-  uint32_t row_step;   // bytes between this thread's successive vectors
-  __device__ __forceinline__ void init(const TI *p, int64_t ld_, int64_t rows_, int64_t K_,
-                                       int64_t r0_) {
-    base = p; ld = ld_; rows = rows_; K = K_; r0 = r0_;
-    if constexpr (BUF) {
-      rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<TI *>(p), (short)0,
-                                               (int)(rows_ * ld_ * (int64_t)sizeof(TI)),
-                                               0x00020000);
-      const int t = threadIdx.x;
-      off0 = (uint32_t)(((r0_ + t / C::KV) * ld_ + (t % C::KV) * C::VE) * (int64_t)sizeof(TI));
-      row_step = (uint32_t)((C::NT / C::KV) * ld_ * (int64_t)sizeof(TI));
-    }
-  }
-  // vector i (0 <= i < count) of the stage starting at k0
-  template <int COUNT>
-  __device__ __forceinline__ void load(int64_t k0, u32x4 (&r)[COUNT]) const {
-    const int t = threadIdx.x;
-    if constexpr (BUF) {
-      const int64_t kk = k0 + (t % C::KV) * C::VE;
-      const bool kin = kk < K;
-      const uint32_t kb = (uint32_t)(k0 * (int64_t)sizeof(TI));
-#pragma unroll
-      for (int i = 0; i < COUNT; ++i) {
-        const bool in = kin && (r0 + t / C::KV + (int64_t)i * (C::NT / C::KV)) < rows;
-        const uint32_t off = in ? off0 + (uint32_t)i * row_step + kb : 0x80000000u;
-        r[i] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rsrc, off, 0, 0));
-      }
-    } else {
-#pragma unroll
-      for (int i = 0; i < COUNT; ++i) {
-        const int v = t + i * C::NT;
-        r[i] = load_vec<TI, false>(base, ld, r0 + v / C::KV, rows, k0 + (v % C::KV) * C::VE, K);
-      }
-    }
-  }
-};
-
-template <class C>
-__device__ __forceinline__ void store_stage(char *stage, const u32x4 (&ra)[C::AV],
-                                            const u32x4 (&rb)[C::BV]) {
-  const int t = threadIdx.x;
-#pragma unroll
-  for (int i = 0; i < C::AV; ++i) {
-    const int v = t + i * C::NT;
-    *reinterpret_cast<u32x4 *>(stage + (v / C::KV) * C::PITCH + (v % C::KV) * 16) = ra[i];
-  }
-  char *bs = stage + C::BM * C::PITCH;
-#pragma unroll
-  for (int i = 0; i < C::BV; ++i) {
-    const int v = t + i * C::NT;
-    *reinterpret_cast<u32x4 *>(bs + (v / C::KV) * C::PITCH + (v % C::KV) * 16) = rb[i];
-  }
-}
-
 template <typename TI>
 __device__ __forceinline__ void mfma_slab(const u32x4 &a, const u32x4 &b,
                                           floatx16 &acc);
@@ -197,26 +98,6 @@ __device__ __forceinline__ void mfma_slab<bf16>(const u32x4 &a, const u32x4 &b,
                                                 floatx16 &acc) {
   acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
       __builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), acc, 0, 0, 0);
-}
-
-template <>
-__device__ __forceinline__ void mfma_slab<float>(const u32x4 &a, const u32x4 &b,
-                                                 floatx16 &acc) {
-#pragma unroll
-  for (int j = 0; j < 4; ++j)
-    acc = __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(a[j]),
-                                               __uint_as_float(b[j]), acc, 0, 0, 0);
-}
-
-template <class C>
-__device__ __forceinline__ void read_operands(const char *as, const char *bs, int kg,
-                                              u32x4 (&a)[C::TM], u32x4 (&b)[C::TN]) {
-#pragma unroll
-  for (int i = 0; i < C::TM; ++i)
-    a[i] = *reinterpret_cast<const u32x4 *>(as + i * 32 * C::PITCH + kg * 32);
-#pragma unroll
-  for (int j = 0; j < C::TN; ++j)
-    b[j] = *reinterpret_cast<const u32x4 *>(bs + j * 32 * C::PITCH + kg * 32);
 }
 
 template <class C>
@@ -245,30 +126,6 @@ __device__ __forceinline__ void interleave_hint() {
   for (int r = 0; r < kReads; ++r) {
     __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);     // 1 DS read
     __builtin_amdgcn_sched_group_barrier(0x008, kPer, 0);  // kPer MFMAs
-  }
-}
-
-template <class C>
-__device__ __forceinline__ void compute_stage(const char *stage, int wm, int wn,
-                                              floatx16 (&acc)[C::TM][C::TN]) {
-  const int l = threadIdx.x & 63;
-  const char *as = stage + (wm * C::WTM + (l & 31)) * C::PITCH + (l >> 5) * 16;
-  const char *bs = stage + (C::BM + wn * C::WTN + (l & 31)) * C::PITCH + (l >> 5) * 16;
-  // operands double-buffered across the four 32-byte k-groups of a stage
-  u32x4 a0[C::TM], b0[C::TN], a1[C::TM], b1[C::TN];
-  read_operands<C>(as, bs, 0, a0, b0);
-#pragma unroll
-  for (int kg = 0; kg < 4; kg += 2) {
-    read_operands<C>(as, bs, kg + 1, a1, b1);
-    mfma_block<C>(a0, b0, acc);
-    interleave_hint<C>();
-    if (kg + 2 < 4) {
-      read_operands<C>(as, bs, kg + 2, a0, b0);
-      mfma_block<C>(a1, b1, acc);
-      interleave_hint<C>();
-    } else {
-      mfma_block<C>(a1, b1, acc);
-    }
   }
 }
 
@@ -872,14 +729,215 @@ __device__ __forceinline__ void mainloop_dtl_ops(const OpA &opa, const OpB &opb,
   __syncthreads();
 }
 
+// ---- fp32 operands as three bf16 parts (SplitCfg) ------------------------------
+// A finite fp32 value is the sum of three bf16 values: b1 its leading 8
+// significant bits (truncated, so nothing overflows), b2 the next 8 of the
+// remainder (rounded) and b3 what is left (exact).  The product of two values
+// is taken as b1 c1 + (b1 c2 + b2 c1 + b1 c3 + b3 c1 + b2 c2); what is left
+// out is below 2^-24 of it, with either sign.  The six products run on
+// v_mfma_f32_16x16x32_bf16, b1 c1 into one accumulator and the five small ones
+// into another (their roundings are then below the first's by 2^-7), added at
+// the end.  Each MFMA adds 32 products to the accumulator with fewer fp32
+// roundings than the fp32 MFMA's one per two k.
+//
+// Against 64 bits (norm-wise relative error, 512 x 512 outputs of N(0, 1)
+// operands / of their absolute values), fp32 MFMAs -> this:
+//   K 64: 1.4e-7 / 1.2e-7 -> 5.4e-8 / 5.2e-8; K 384: 3.5e-7 / 2.7e-7 -> 1.1e-7 /
+//   1.0e-7; K 2048: 8.1e-7 / 7.0e-7 -> 2.7e-7 / 2.5e-7; K 32000: 3.2e-6 / 2.8e-6
+//   -> 1.1e-6 / 9.9e-7.
+// Rate on fp32 operands: 4096^3 117 -> 192 TFLOP/s, M 32000 N 512 K 384 97 -> 172
+// (the fp32 matrix rate is 157 at most).
+//
+// A block tile of BM x BN, 8 wavefronts of 64 x 64; a stage is 32 k of every
+// tile row, loaded into registers as fp32 while the stage before is
+// multiplied, split there and written to LDS as three planes of 64-byte rows
+// (two stage buffers).  Bound by the matrix pipes: 96 MFMAs per wavefront and
+// stage against 24 LDS reads, 9 LDS writes and ~190 vector instructions.
+template <int BM_, int BN_, int WM_, int WN_>
+struct SplitCfg {
+  using TI = float;
+  static constexpr bool DTL = false;
+  static constexpr int BM = BM_, BN = BN_, WM = WM_, WN = WN_;
+  static constexpr int NT = WM * WN * 64;
+  static constexpr int WTM = BM / WM, WTN = BN / WN;
+  static constexpr int TM = WTM / 32, TN = WTN / 32;
+  static constexpr int VE = 4;                    // fp32 per 16-byte vector
+  static constexpr int BK = 32;                   // k per stage
+  static constexpr int ROW = BK * 2;              // LDS row of one part, bytes
+  static constexpr int PLANE = (BM + BN) * ROW;   // one part of a stage
+  static constexpr int STAGE = 3 * PLANE;
+  static constexpr int LDS_BYTES = 2 * STAGE;
+  static constexpr int RPP = NT / 4;              // tile rows per pass (4 threads a row)
+  static constexpr int AP = BM / RPP, BP = BN / RPP;  // passes over A, B rows
+  static_assert(BM % RPP == 0 && BN % RPP == 0, "loader passes");
+  static_assert(WTM == 64 && WTN == 64, "64 x 64 per wavefront");
+};
+
+// The 16-byte k-vector kv (0..3) of LDS row `row` sits in slot
+// split_slot(row, kv): an operand read of a wavefront touches rows r (lane
+// % 16) at kv lane / 16, and this puts the 16 lanes that a ds_read_b128
+// serves together into 16 different 16-byte columns of the banks.
+__device__ __forceinline__ int split_slot(int row, int kv) { return kv ^ ((row >> 2) & 2); }
+
+// 8 fp32 (two 16-byte vectors) -> the three parts, 8 bf16 each
+__device__ __forceinline__ void split8(const u32x4 (&x)[2], u32x4 (&part)[3]) {
+  typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+#pragma unroll
+  for (int p = 0; p < 4; ++p) {  // pairs
+    const uint32_t u0 = x[p >> 1][2 * (p & 1)], u1 = x[p >> 1][2 * (p & 1) + 1];
+    const float f0 = __uint_as_float(u0), f1 = __uint_as_float(u1);
+    const uint32_t h0 = u0 & 0xffff0000u, h1 = u1 & 0xffff0000u;
+    // an infinity is its own first part, with nothing left
+    const float r0 = (u0 & 0x7fffffffu) == 0x7f800000u ? 0.f : f0 - __uint_as_float(h0);
+    const float r1 = (u1 & 0x7fffffffu) == 0x7f800000u ? 0.f : f1 - __uint_as_float(h1);
+    part[0][p] = (h0 >> 16) | h1;
+    const bf16x2 m = {static_cast<__bf16>(r0), static_cast<__bf16>(r1)};
+    const uint32_t mb = __builtin_bit_cast(uint32_t, m);
+    part[1][p] = mb;
+    const bf16x2 l = {static_cast<__bf16>(r0 - __uint_as_float(mb << 16)),
+                      static_cast<__bf16>(r1 - __uint_as_float(mb & 0xffff0000u))};
+    part[2][p] = __builtin_bit_cast(uint32_t, l);
+  }
+}
+
+// One operand's rows of a block tile: thread t loads k 8 (t % 4) .. + 7 of tile
+// rows t / 4 + RPP i, i < NP.  BUF: through a buffer resource (rows past the
+// matrix and k past K read as zero by an out-of-range offset; K % 4 == 0,
+// aligned rows, under 2 GiB); else element-wise.
+template <class C, int NP, bool BUF>
+struct SplitOperand {
+  const float *base;
+  int64_t ld, rows, K, r0;
+  __amdgpu_buffer_rsrc_t rsrc;
+  uint32_t off0, step;
+  __device__ __forceinline__ void init(const float *p, int64_t ld_, int64_t rows_, int64_t K_,
+                                       int64_t r0_) {
+    base = p; ld = ld_; rows = rows_; K = K_; r0 = r0_ + threadIdx.x / 4;
+    if constexpr (BUF) {
+      rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(p), (short)0,
+                                               (int)(rows_ * ld_ * 4), 0x00020000);
+      off0 = (uint32_t)((r0 * ld_ + 8 * (threadIdx.x % 4)) * 4);
+      step = (uint32_t)(C::RPP * ld_ * 4);
+    }
+  }
+  __device__ __forceinline__ void load(int64_t k0, u32x4 (&v)[NP][2]) const {
+    const int64_t k = k0 + 8 * (threadIdx.x % 4);
+#pragma unroll
+    for (int i = 0; i < NP; ++i)
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        if constexpr (BUF) {
+          const bool in = r0 + i * C::RPP < rows && k + 4 * h < K;
+          const uint32_t o = off0 + (uint32_t)i * step + (uint32_t)(k0 * 4) + 16 * h;
+          v[i][h] = __builtin_bit_cast(
+              u32x4, __builtin_amdgcn_raw_buffer_load_b128(rsrc, in ? o : 0x80000000u, 0, 0));
+        } else {
+          v[i][h] = load_vec<float, false>(base, ld, r0 + i * C::RPP, rows, k + 4 * h, K);
+        }
+      }
+  }
+  // the three parts into the stage's planes, tile rows from `row0` of a plane
+  __device__ __forceinline__ void store(const u32x4 (&v)[NP][2], char *stage, int row0) const {
+#pragma unroll
+    for (int i = 0; i < NP; ++i) {
+      u32x4 part[3];
+      split8(v[i], part);
+      const int row = threadIdx.x / 4 + i * C::RPP;
+      char *dst = stage + (row0 + row) * C::ROW + split_slot(row, threadIdx.x % 4) * 16;
+#pragma unroll
+      for (int q = 0; q < 3; ++q) *reinterpret_cast<u32x4 *>(dst + q * C::PLANE) = part[q];
+    }
+  }
+};
+
+// The wavefront's 16x16x32 operands of one part: rows of A as read_kgroup16
+// takes them (bits 2 and 3 of lane % 16 swapped), rows of B in order.
+template <class C>
+__device__ __forceinline__ void split_read_a(const char *plane, int wm, u32x4 (&a)[2 * C::TM]) {
+  const int l = threadIdx.x & 63, i16 = l & 15;
+  const int r = (i16 & 3) | ((i16 & 4) << 1) | ((i16 & 8) >> 1);
+  const char *p = plane + (wm * C::WTM + r) * C::ROW + split_slot(r, l >> 4) * 16;
+#pragma unroll
+  for (int i = 0; i < 2 * C::TM; ++i) a[i] = *reinterpret_cast<const u32x4 *>(p + i * 16 * C::ROW);
+}
+template <class C>
+__device__ __forceinline__ void split_read_b(const char *plane, int wn, u32x4 (&b)[2 * C::TN]) {
+  const int l = threadIdx.x & 63, r = l & 15;
+  const char *p = plane + (C::BM + wn * C::WTN + r) * C::ROW + split_slot(r, l >> 4) * 16;
+#pragma unroll
+  for (int j = 0; j < 2 * C::TN; ++j) b[j] = *reinterpret_cast<const u32x4 *>(p + j * 16 * C::ROW);
+}
+
+template <class C, bool BUF, bool ZERO>
+__device__ __forceinline__ void mainloop_split(const float *A, int64_t lda, const float *B,
+                                               int64_t ldb, int64_t M, int64_t N, int64_t K,
+                                               int64_t m0, int64_t n0, char *smem,
+                                               floatx16 (&acc)[C::TM][C::TN]) {
+  const int w = threadIdx.x >> 6, wm = w / C::WN, wn = w % C::WN;
+  floatx16 low[C::TM][C::TN];
+#pragma unroll
+  for (int i = 0; i < C::TM; ++i)
+#pragma unroll
+    for (int j = 0; j < C::TN; ++j) {
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        low[i][j][r] = 0.f;
+        if constexpr (ZERO) acc[i][j][r] = 0.f;
+      }
+      if constexpr (!ZERO) acc_swap16(acc[i][j]);
+    }
+  SplitOperand<C, C::AP, BUF> opa;
+  SplitOperand<C, C::BP, BUF> opb;
+  opa.init(A, lda, M, K, m0);
+  opb.init(B, ldb, N, K, n0);
+  const int nk = (int)((K + C::BK - 1) / C::BK);
+  u32x4 ra[C::AP][2], rb[C::BP][2];
+  opa.load(0, ra);
+  opb.load(0, rb);
+  opa.store(ra, smem, 0);
+  opb.store(rb, smem, C::BM);
+  opa.load(C::BK, ra);  // past K: zeros
+  opb.load(C::BK, rb);
+  __syncthreads();
+  for (int kt = 0; kt < nk; ++kt) {
+    const char *cur = smem + (kt & 1) * C::STAGE;
+    char *nxt = smem + ((kt + 1) & 1) * C::STAGE;
+    u32x4 a1[2 * C::TM], a2[2 * C::TM], a3[2 * C::TM], b[2 * C::TN];
+    split_read_a<C>(cur, wm, a1);
+    split_read_b<C>(cur, wn, b);
+    // the next stage out of the registers, the one after into them
+    opa.store(ra, nxt, 0);
+    opb.store(rb, nxt, C::BM);
+    opa.load((int64_t)(kt + 2) * C::BK, ra);
+    opb.load((int64_t)(kt + 2) * C::BK, rb);
+    mfma_block16<C>(a1, b, acc);
+    split_read_a<C>(cur + C::PLANE, wm, a2);
+    mfma_block16<C>(a2, b, low);
+    split_read_a<C>(cur + 2 * C::PLANE, wm, a3);
+    mfma_block16<C>(a3, b, low);
+    split_read_b<C>(cur + C::PLANE, wn, b);
+    mfma_block16<C>(a1, b, low);
+    mfma_block16<C>(a2, b, low);
+    split_read_b<C>(cur + 2 * C::PLANE, wn, b);
+    mfma_block16<C>(a1, b, low);
+    __syncthreads();
+  }
+#pragma unroll
+  for (int i = 0; i < C::TM; ++i)
+#pragma unroll
+    for (int j = 0; j < C::TN; ++j) {
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        // an infinite operand makes b1 c1 what the fp32 product is, and the
+        // small products inf * 0: those are left out there
+        const float hi = acc[i][j][r];
+        acc[i][j][r] = __builtin_isfinite(hi) ? hi + low[i][j][r] : hi;
+      }
+      acc_swap16(acc[i][j]);
+    }
+}
+
 // Full K loop for the block tile at (m0, n0).  `smem` holds C::LDS_BYTES.
-// With C::PF == 2, global loads run two K-stages ahead of the MFMAs in two
-// alternating register sets (while stage k is multiplied out of LDS, stage
-// k+1 sits in registers waiting for the other LDS buffer and stage k+2 is in
-// flight): a small wave tile's compute stage is too short to hide HBM/MALL
-// latency alone.  With C::PF == 1 one register set holds stage k+1 while
-// stage k is computed: large wave tiles (and a second wavefront per SIMD)
-// cover the latency, and a second set would not fit beside the accumulators.
 // Ends with a barrier, so the caller may reuse smem for its epilogue.
 // ZERO: start from acc = 0; otherwise the caller has loaded acc (C += A B^T).
 template <class C, bool BUF, bool ZERO = true>
@@ -888,72 +946,10 @@ __device__ __forceinline__ void mainloop(const typename C::TI *A, int64_t lda,
                                          int64_t M, int64_t N, int64_t K,
                                          int64_t m0, int64_t n0, char *smem,
                                          floatx16 (&acc)[C::TM][C::TN]) {
-  if constexpr (C::DTL) {
+  if constexpr (C::DTL)
     mainloop_dtl<C, BUF, ZERO>(A, lda, B, ldb, M, N, K, m0, n0, smem, acc);
-    return;
-  } else {
-  const int w = threadIdx.x >> 6;
-  const int wm = w / C::WN, wn = w % C::WN;
-  if constexpr (ZERO) {
-#pragma unroll
-    for (int i = 0; i < C::TM; ++i)
-#pragma unroll
-      for (int j = 0; j < C::TN; ++j)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
-  }
-
-  Operand<C, BUF> opa, opb;
-  opa.init(A, lda, M, K, m0);
-  opb.init(B, ldb, N, K, n0);
-  const int64_t nk = (K + C::BK - 1) / C::BK;
-  char *const lds0 = smem;
-  char *const lds1 = smem + C::STAGE;
-  if constexpr (C::PF == 2) {
-    u32x4 ra0[C::AV], rb0[C::BV], ra1[C::AV], rb1[C::BV];
-    opa.load(0, ra0);
-    opb.load(0, rb0);
-    store_stage<C>(lds0, ra0, rb0);
-    if (nk > 1) { opa.load(C::BK, ra1); opb.load(C::BK, rb1); }
-    if (nk > 2) { opa.load(2 * C::BK, ra0); opb.load(2 * C::BK, rb0); }
-    __syncthreads();
-    for (int64_t kt = 0; kt < nk; kt += 2) {
-      // even stage kt in lds0; stage kt+1 in (ra1, rb1); stage kt+2 in (ra0, rb0)
-      compute_stage<C>(lds0, wm, wn, acc);
-      if (kt + 1 < nk) {
-        store_stage<C>(lds1, ra1, rb1);
-        if (kt + 3 < nk) { opa.load((kt + 3) * C::BK, ra1); opb.load((kt + 3) * C::BK, rb1); }
-      }
-      __syncthreads();
-      if (kt + 1 >= nk) break;
-      // odd stage kt+1 in lds1; stage kt+2 in (ra0, rb0); stage kt+3 in (ra1, rb1)
-      compute_stage<C>(lds1, wm, wn, acc);
-      if (kt + 2 < nk) {
-        store_stage<C>(lds0, ra0, rb0);
-        if (kt + 4 < nk) { opa.load((kt + 4) * C::BK, ra0); opb.load((kt + 4) * C::BK, rb0); }
-      }
-      __syncthreads();
-    }
-  } else {
-    u32x4 ra[C::AV], rb[C::BV];
-    opa.load(0, ra);
-    opb.load(0, rb);
-    store_stage<C>(lds0, ra, rb);
-    if (nk > 1) { opa.load(C::BK, ra); opb.load(C::BK, rb); }
-    __syncthreads();
-    for (int64_t kt = 0; kt < nk; ++kt) {
-      // stage kt in LDS buffer kt&1; stage kt+1 in (ra, rb)
-      char *const cur = (kt & 1) ? lds1 : lds0;
-      char *const nxt = (kt & 1) ? lds0 : lds1;
-      compute_stage<C>(cur, wm, wn, acc);
-      if (kt + 1 < nk) {
-        store_stage<C>(nxt, ra, rb);
-        if (kt + 2 < nk) { opa.load((kt + 2) * C::BK, ra); opb.load((kt + 2) * C::BK, rb); }
-      }
-      __syncthreads();
-    }
-  }
-  }
+  else
+    mainloop_split<C, BUF, ZERO>(A, lda, B, ldb, M, N, K, m0, n0, smem, acc);
 }
 
 // Output tile of a one-dimensional grid's block b, for `total` = tiles_m *

@@ -557,14 +557,14 @@ inline int launch_zero16(void *p, int64_t ld, int64_t rows, int64_t cols, hipStr
 
 // bf16: 256x256 block tiles, 8 wavefronts of 128x64 (two per SIMD, so one
 // wavefront's LDS waits and epilogue overlap the other's MFMAs), operands
-// copied global -> LDS directly in 64-wide K-stages, two stage buffers; f32
-// (correctness path): 128x128 tiles staged through registers.
+// copied global -> LDS directly in 64-wide K-stages, two stage buffers; f32:
+// 256x128 tiles, split into bf16 parts on the way to LDS.
 template <typename TI>
 struct MainCfgT;
 template <>
 struct MainCfgT<bf16> { using type = gemm::DCfg<256, 256, 2, 4, 2, 64>; };
 template <>
-struct MainCfgT<float> { using type = Cfg<float, 128, 128, 2, 2>; };
+struct MainCfgT<float> { using type = SplitCfg<256, 128, 4, 2>; };
 template <typename TI>
 using MainCfg = typename MainCfgT<TI>::type;
 // 192 rows (B N-major) or columns (B K-contiguous) in the place of 256, for an
