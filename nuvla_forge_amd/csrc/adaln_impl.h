@@ -1100,25 +1100,32 @@ inline unsigned fwd_grid(const Plan &pl, int64_t M) {
 constexpr bool kFwdNT = true;
 constexpr bool kBwdNT = true;
 
-// The batched forward (adaln_fwd_batch_kernel) takes RB rows per step: 4 with
-// one 8-element chunk per thread, 2 with two; 16-bit x and y only (fp32 rows
-// would not fit the registers), and only when every row group's rows lie in
-// one sample and split into whole batches.  Measured at bf16 [8192, 1024]:
-// 10.5 us against 12.3 us for the one-row-at-a-time kernel, bit-identical.
+// The batched forward (adaln_fwd_batch_kernel) takes RB rows per step: in 16
+// bits 4 with one 8-element chunk per thread and 2 with two, for fp32 x 4; only
+// when every row group's rows lie in one sample and split into whole batches,
+// and for fp32 x only where the loads are hinted (beyond the Infinity Cache).
+// The same bits as the one-row-at-a-time kernel in 16 bits, the same to fp32
+// rounding in fp32.  Measured: bf16 [8192, 1024]
+// 10.5 us against 12.3; x fp32, y bf16, forward + backward, [16, 2048, 2048]
+// 4.81 TB/s against 4.38, [32, 512, 4096] 4.75 against 4.28, but in the cache
+// [32, 512, 768] 4.33 against 4.58 and [8, 1024, 1024] level.
 template <typename TX, typename TY, int K>
 constexpr int fwd_batch_rows() {
-  return (sizeof(TX) == 2 && sizeof(TY) == 2) ? (K == 1 ? 4 : 2) : 1;
+  return (sizeof(TX) == 2 && sizeof(TY) == 2) ? (K == 1 ? 4 : 2) : 4;
 }
 template <typename TX, typename TY, bool VEC, int WPR, int K>
 int launch_fwd_t(const FwdArgs &a, const Plan &pl, hipStream_t s) {
   using S = FwdShape<WPR, fwd_min_block<K>()>;  // the shape of both kernels below
   constexpr int RB = fwd_batch_rows<TX, TY, K>();
-  if constexpr (VEC && RB > 1) {
-    if (a.rows_per_group % RB == 0 && a.T % a.rows_per_group == 0) {
-      if (nt_loads_for(a.M * a.N * (int64_t)(sizeof(TX) + sizeof(TY))))
+  // fp32 rows of more than 512 threads would not fit the registers
+  if constexpr (VEC && (sizeof(TX) == 2 || S::BLK <= 512)) {
+    const bool ntl = nt_loads_for(a.M * a.N * (int64_t)(sizeof(TX) + sizeof(TY)));
+    if (a.rows_per_group % RB == 0 && a.T % a.rows_per_group == 0 &&
+        (sizeof(TX) == 2 || ntl)) {
+      if (ntl)
         adaln_fwd_batch_kernel<TX, TY, K, WPR, VEC, kFwdNT, RB, true>
             <<<fwd_grid<S>(pl, a.M), S::BLK, 0, s>>>(a);
-      else
+      else if constexpr (sizeof(TX) == 2)
         adaln_fwd_batch_kernel<TX, TY, K, WPR, VEC, kFwdNT, RB, false>
             <<<fwd_grid<S>(pl, a.M), S::BLK, 0, s>>>(a);
       return check_launch("nf_adaln_fwd");

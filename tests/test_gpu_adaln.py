@@ -148,6 +148,34 @@ def test_adaln_backward_over_many_samples(cuda, xd, yd, b, t, n):
         assert torch.equal(v, grads[k]), f"d{k} alone differs"
 
 
+@pytest.mark.parametrize("yd,b,t,n", [
+    (torch.bfloat16, 15, 4096, 1024),  # one chunk a lane
+    (torch.float32, 4, 4096, 2568),    # two chunks, a partial last one
+    (torch.float32, 3, 2048, 8192),    # eight wavefronts a row
+])
+def test_adaln_forward_beyond_the_cache_fp32(cuda, yd, b, t, n):
+    """fp32 rows of more than 320 MiB of x and y go in batches of four; each
+    sample alone goes a row at a time: the same h, and out to its rounding."""
+    note(f"adaln fp32 forward beyond the cache {yd} b={b} t={t} n={n}")
+    g = torch.Generator(device=cuda).manual_seed(5)
+    draw = lambda *s: torch.randn(*s, device=cuda, generator=g)  # noqa: E731
+    x, y, w = draw(b * t, n), draw(b * t, n).to(yd), draw(n)
+    assert x.numel() * (4 + y.element_size()) > 320 << 20
+    gate, scale, shift = draw(b, n).to(yd), draw(b, n).to(yd), draw(b, n).to(yd)
+    h, out = fused_adaln_residual_rmsnorm(x, y, gate, w, scale, shift, tokens_per_sample=t)
+    for k in range(b):
+        r, c = slice(k * t, (k + 1) * t), slice(k, k + 1)
+        h1, out1 = fused_adaln_residual_rmsnorm(x[r], y[r], gate[c], w, scale[c], shift[c],
+                                                tokens_per_sample=t)
+        assert torch.equal(h[r], h1)
+        # The sum of squares may round differently (16 products a lane, 6 tree
+        # steps, 8 wavefronts: 30 roundings of 2^-24 on each side at most, half of
+        # it in rstd), and rstd, two products and the last add once each: 34 units
+        # of 2^-24 of the modulated term and of the shift beside it.
+        size = (out1 - shift[c].float()).abs() + shift[c].float().abs()
+        assert ((out[r] - out1).abs() <= 34 * 2.0 ** -24 * size).all()
+
+
 def test_cfg2_bf16_and_bitwise_deterministic_backward(cuda):
     note("adaln cfg2 bf16 [8,1024,1024] x10 backward")
     b, t, n = 8, 1024, 1024
