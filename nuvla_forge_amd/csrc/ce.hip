@@ -743,44 +743,43 @@ __global__ __launch_bounds__(256) void ce_scatter_dh_kernel(const float *__restr
 // ---------------------------------------------------------------------------
 
 // K split of a chunk's dH product.  The launch holding a chunk's gradient
-// products has the dW blocks (K = the chunk's rows, crows) and the dH blocks
-// (K = V, long); dH is split into S slices to balance them: S minimises the
-// launch's makespan, max(longest block, total work / 256 CUs), plus the
-// write and read of the S fp32 slices, all in units of one 64-deep K stage of
-// a 256 x 256 tile (~2 us per CU at ~1.1 PFLOP/s, against ~5 TB/s of HBM).
-// At cfg4 in one chunk (3687 rows) it does not split (128 dH blocks of K
-// 32000 beside 1000 dW blocks of K 3687 balance by themselves): measured
-// against forcing slices of at most 2048 / 4096 / 8192 / 16384 (16 / 8 / 4 /
-// 2 slices), 1.64-1.66 ms against 1.85 / 1.77-1.80 / 1.72-1.74 / 1.67-1.69 ms
-// per fwd+bwd: the extra fp32 slice traffic costs more than shorter blocks
-// gain.  (This holds with the long job's blocks spread over all XCDs, see
-// gemm_store_kernel.)
+// products has the dW blocks (K = the chunk's rows) and the dH blocks
+// (K = V, long); dH is split into S slices so that the two kinds of blocks
+// fill the 256 CUs to the same end: S minimises the launch's makespan, plus
+// the write and (partly hidden) read of the S fp32 slices (~5 TB/s).  Block times from
+// timestamps in the launch (us): a 64-deep stage of a 256 x 256 or 256 x 192
+// tile 1.3-1.8 with K-contiguous operands and 1.8-2.0 with the N-major E
+// (single), a 32-deep stage of the fp32 256 x 128 tile ~2; on top of its stages
+// ~12 for a dW block (the accumulator's rows read before, stored after) and ~8
+// for a dH block.  dcols: tile extent along D (C::BN, or 192).
+// Swept (forward + backward): M 12289 D 384 V 50001 2.35 ms with 8 slices (8 of
+// the 392 dW blocks are left to a last round of their own), 2.29 with 7, 2.45
+// with 12-16; M 300 D 1024 V 128256 557 us with 16, 578 with 14 or 18, 647 with
+// 8; M 4096 D 2048 V 32000 1.39 ms unsplit, 1.41 with 2, 1.51 with 8.
 struct Split {
   int S;
   int64_t kslice;
 };
-// dcols: tile extent along D (C::BN, or 192: then a stage is 3/4 the work).
 template <class C>
-inline Split dh_split(int64_t crows, int64_t D, int64_t V, int64_t ldp, bool single,
+inline Split dh_split(int64_t rows, int64_t D, int64_t V, int64_t ldp, bool single,
                       int64_t dcols) {
   const int64_t tn = (D + dcols - 1) / dcols;
-  const double tw = (double)((V + C::BM - 1) / C::BM * tn);
-  const double th = (double)((crows + C::BM - 1) / C::BM * tn);
-  // the N-major dW product (single) issues 8 LDS reads per 8 MFMAs against
-  // 6: ~12% longer stages measured at K = 2048 / 4096
-  const double kw = (double)crows / C::BK * (single ? 1.12 : 1.0);
-  const double stage_s = 2e-6 * (double)dcols / C::BN, hbm_bps = 5e12;
+  const int64_t nw = (V + C::BM - 1) / C::BM * tn;
+  const int64_t nh = (rows + C::BM - 1) / C::BM * tn;
+  const double nt = sizeof(typename C::TI) == 2 ? 1.65 : 2.0;
+  const double lw = (double)((rows + C::BK - 1) / C::BK) * (single ? 1.9 : nt) + 12.0;
   Split best{1, ldp};
   double best_t = -1.0;
-  for (int S = 1; S <= 64; ++S) {
+  for (int S = 1; S <= 64; S += S < 16 ? 1 : 4) {
     const int64_t ks = round_up((ldp + S - 1) / S, C::BK);
     const int64_t se = (ldp + ks - 1) / ks;
-    const double kh = (double)ks / C::BK;
-    const double work = tw * kw + th * (double)se * kh;
-    double t = work / 256.0;
-    if (kh > t) t = kh;
-    if (kw > t) t = kw;
-    if (se > 1) t += 2.0 * se * crows * D * 4.0 / hbm_bps / stage_s;
+    const double lh = (double)(ks / C::BK) * nt + 8.0;
+    double t = lh >= lw ? two_job_makespan(nh * se, lh, nw, lw)
+                        : two_job_makespan(nw, lw, nh * se, lh);
+    // the XCDs take contiguous ranges of a job's blocks: slices that are not
+    // whole ranges share no operands there
+    if (se % 8 != 0 && 8 % se != 0) t *= 1.04;
+    if (se > 1) t += 1.5 * (double)(se * rows * D) * 4.0 / 5e12 * 1e6;
     if (best_t < 0 || t < best_t - 1e-9) {
       best_t = t;
       best = {(int)se, ks};
@@ -819,7 +818,7 @@ inline int64_t line_stride(int64_t n, size_t es) {
 }
 
 template <typename TI>
-inline Plan make_plan(int64_t M, int64_t D, int64_t V, int64_t chunk_rows) {
+inline Plan plan_shape(int64_t M, int64_t D, int64_t V, int64_t chunk_rows) {
   using C = MainCfg<TI>;
   const size_t es = sizeof(TI);
   Plan P{};
@@ -863,7 +862,7 @@ inline Plan make_plan(int64_t M, int64_t D, int64_t V, int64_t chunk_rows) {
   // With E held once D is a tile extent of both gradient products (rows of
   // dW^T, columns of dH); a 192 tile reads ~6% more operand per product.
   P.d192 = P.single && round_up(D, 192) * 1.06 < round_up(D, 256);
-  P.split = dh_split<C>(P.crows, D, V, P.ldp, P.single, P.d192 ? 192 : C::BN);
+  P.split = dh_split<C>(P.crows < M ? P.crows : M, D, V, P.ldp, P.single, P.d192 ? 192 : C::BN);
   const size_t part = P.split.S > 1 ? (size_t)P.split.S * P.crows * D * sizeof(float) : 0;
   size_t o = 0;
   auto take = [&](size_t bytes) { const size_t at = o; o = align256(o + bytes); return at; };
@@ -891,6 +890,20 @@ inline Plan make_plan(int64_t M, int64_t D, int64_t V, int64_t chunk_rows) {
   P.b_part = take(part);
   P.b_total = o;
   return P;
+}
+
+// A thread keeps its last shape's plan: the size calls and the launches of
+// every step ask for the same one.
+template <typename TI>
+inline Plan make_plan(int64_t M, int64_t D, int64_t V, int64_t chunk_rows) {
+  struct Kept {
+    int64_t M, D, V, chunk_rows;
+    Plan P;
+  };
+  static thread_local Kept kept{0, 0, 0, 0, {}};
+  if (kept.M != M || kept.D != D || kept.V != V || kept.chunk_rows != chunk_rows)
+    kept = {M, D, V, chunk_rows, plan_shape<TI>(M, D, V, chunk_rows)};
+  return kept.P;
 }
 
 // Pointers into the state.

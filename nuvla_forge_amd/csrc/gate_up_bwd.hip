@@ -224,28 +224,10 @@ __global__ __launch_bounds__(kSumThreads) void gate_up_reduce_kernel(Sums p) {
 // K splits of the launch.  nx dx tiles of kx stages and nw dW tiles of kw
 // stages run on 256 CUs, one block each, the longer blocks first; a block
 // also costs ~4 stages of prologue and epilogue, and a split product the
-// write and read of its fp32 slices (stages of ~1.8 us against ~5 TB/s).  The
-// makespan is the first time by which the CUs can have taken every short
-// block beside or after the long ones.
+// write and read of its fp32 slices (stages of ~1.8 us against ~5 TB/s).
 struct Split {
   int sx, sw;
 };
-inline double makespan(int64_t n1, double l1, int64_t n2, double l2) {
-  const int64_t cus = 256;
-  const int64_t r = n1 / cus, rest = n1 % cus;  // whole rounds of long blocks
-  double t = n1 ? (double)(rest ? r + 1 : r) * l1 : 0.0;
-  for (int it = 0; it < 4096; ++it) {
-    const double ta = t - (double)r * l1, tb = ta - l1;
-    const int64_t cap = (cus - rest) * (int64_t)(ta / l2 + 1e-9) +
-                        (tb > 0 ? rest * (int64_t)(tb / l2 + 1e-9) : 0);
-    if (cap >= n2) return t;
-    // the next time another short block can have ended
-    const double fa = ((int64_t)(ta / l2 + 1e-9) + 1) * l2;
-    const double fb = rest ? l1 + ((int64_t)(tb > 0 ? tb / l2 + 1e-9 : 0) + 1) * l2 : fa;
-    t = (double)r * l1 + (fa < fb ? fa : fb);
-  }
-  return t;
-}
 inline Split pick_split(int64_t M, int64_t D, int64_t H, bool want_x, int want_w) {
   const int64_t td = (D + C::BM - 1) / C::BM;
   const int64_t nx = want_x ? td * ((M + C::BN - 1) / C::BN) : 0;
@@ -257,7 +239,8 @@ inline Split pick_split(int64_t M, int64_t D, int64_t H, bool want_x, int want_w
   for (int sx = 1; sx <= 8 && (sx == 1 || (want_x && kx / sx >= 4)); ++sx)
     for (int sw = 1; sw <= 32 && (sw == 1 || (want_w && kw / sw >= 4)); ++sw) {
       const double lx = (double)((kx + sx - 1) / sx) + over, lw = (double)((kw + sw - 1) / sw) + over;
-      double t = lx >= lw ? makespan(nx * sx, lx, nw * sw, lw) : makespan(nw * sw, lw, nx * sx, lx);
+      double t = lx >= lw ? gemm::two_job_makespan(nx * sx, lx, nw * sw, lw)
+                          : gemm::two_job_makespan(nw * sw, lw, nx * sx, lx);
       if (sx > 1) t += 2.0 * sx * (double)M * D * 4 * per_byte;
       if (sw > 1) t += 2.0 * sw * want_w * (double)H * D * 4 * per_byte;
       if (best_t < 0 || t < best_t * 0.999) {
@@ -272,7 +255,17 @@ struct Layout {
   Split sp;
   size_t off_x, off_g, off_u, total;
 };
+// A thread keeps its last shape's layout: the workspace call and the launch
+// of every step ask for the same one.
 inline Layout layout(int64_t M, int64_t D, int64_t H, bool x, bool g, bool u) {
+  struct Kept {
+    int64_t M, D, H;
+    int want;
+    Layout L;
+  };
+  static thread_local Kept kept{0, 0, 0, 0, {}};
+  const int want = (int)x + 2 * (int)g + 4 * (int)u;
+  if (kept.M == M && kept.D == D && kept.H == H && kept.want == want) return kept.L;
   Layout L{};
   L.sp = pick_split(M, D, H, x, (int)g + (int)u);
   size_t o = 0;
@@ -281,6 +274,7 @@ inline Layout layout(int64_t M, int64_t D, int64_t H, bool x, bool g, bool u) {
   L.off_g = take(g && L.sp.sw > 1 ? (size_t)L.sp.sw * H * D * sizeof(float) : 0);
   L.off_u = take(u && L.sp.sw > 1 ? (size_t)L.sp.sw * H * D * sizeof(float) : 0);
   L.total = o;
+  kept = {M, D, H, want, L};
   return L;
 }
 

@@ -575,6 +575,27 @@ using Cols192Cfg = gemm::DCfg<256, 192, 4, 2, 2, 64>;
 inline int64_t round_up(int64_t x, int64_t m) { return (x + m - 1) / m * m; }
 inline size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
 
+// The time by which 256 CUs, one block each, have run n1 blocks of l1 and then
+// n2 of l2 <= l1, taken in that order as CUs come free: at the earliest the
+// work over the CUs, then the first time by which enough short blocks can
+// have ended beside or after the long ones.
+inline double two_job_makespan(int64_t n1, double l1, int64_t n2, double l2) {
+  constexpr int64_t cus = 256;
+  const int64_t full = n1 / cus, rest = n1 % cus;  // whole rounds of long blocks
+  const double t0 = (double)full * l1;
+  double t = n1 ? (double)(full + (rest ? 1 : 0)) * l1 : 0.0;
+  const double work = ((double)n1 * l1 + (double)n2 * l2) / (double)cus;
+  if (t < work) t = work;
+  for (int it = 0; it < 64; ++it) {
+    const double ta = t - t0, tb = rest ? ta - l1 : -1.0;
+    const int64_t ka = (int64_t)(ta / l2 + 1e-9), kb = tb > 0 ? (int64_t)(tb / l2 + 1e-9) : 0;
+    if ((cus - rest) * ka + rest * kb >= n2) return t;
+    const double fa = (double)(ka + 1) * l2, fb = rest ? l1 + (double)(kb + 1) * l2 : fa;
+    t = t0 + (fa < fb ? fa : fb);  // the next time a short block can have ended
+  }
+  return t;
+}
+
 template <class C>
 GemmJob<typename C::TI> make_job(const typename C::TI *A, int64_t lda, const typename C::TI *B,
                                  int64_t ldb, const float *Cin, void *Cout, int cdt,
