@@ -204,18 +204,28 @@ Tensor rows_bf16(const Tensor &t) {
   return r.stride(-1) == 1 ? r : r.contiguous();
 }
 
+// act = silu(x wg^T) * (x wu^T); a and b (the two products) are written where
+// `save`, for the backward.
+Tensor gate_up_forward(const Tensor &x, const Tensor &wg, const Tensor &wu, bool save, Tensor &a,
+                       Tensor &b) {
+  const int64_t m = x.size(0), d = x.size(1), h = wg.size(0);
+  if (save) a = at::empty({m, h}, x.options());
+  if (save) b = at::empty({m, h}, x.options());
+  Tensor act = at::empty({m, h}, x.options());
+  check(nf_gemm_swiglu(x.data_ptr(), x.stride(0), wg.data_ptr(), wg.stride(0), wu.data_ptr(),
+                       wu.stride(0), ptr(a), ptr(b), act.data_ptr(), h, m, d, h, NF_DTYPE_BF16,
+                       stream_of(x)),
+        "nf_gemm_swiglu");
+  return act;
+}
+
 struct GateUp : torch::autograd::Function<GateUp> {
   static Tensor forward(AutogradContext *ctx, const Tensor &x_in, const Tensor &g_in,
                         const Tensor &u_in) {
     const c10::DeviceGuard guard(x_in.device());
     const Tensor x = rows_bf16(x_in), wg = rows_bf16(g_in), wu = rows_bf16(u_in);
-    const int64_t m = x.size(0), d = x.size(1), h = wg.size(0);
-    Tensor a = at::empty({m, h}, x.options()), b = at::empty({m, h}, x.options());
-    Tensor act = at::empty({m, h}, x.options());
-    check(nf_gemm_swiglu(x.data_ptr(), x.stride(0), wg.data_ptr(), wg.stride(0), wu.data_ptr(),
-                         wu.stride(0), a.data_ptr(), b.data_ptr(), act.data_ptr(), h, m, d, h,
-                         NF_DTYPE_BF16, stream_of(x)),
-          "nf_gemm_swiglu");
+    Tensor a, b;
+    const Tensor act = gate_up_forward(x, wg, wu, true, a, b);
     ctx->save_for_backward({x, wg, wu, a, b});
     ctx->saved_data["dt"] = std::vector<int64_t>{(int64_t)x_in.scalar_type(),
                                                  (int64_t)g_in.scalar_type(),
@@ -362,6 +372,15 @@ PyObject *py_gate_up(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
   for (const Tensor &v : t)
     if (!plain(v, dev) || code_of(v) < 0 || v.dim() != 2 || v.numel() == 0) Py_RETURN_NONE;
   if (t[1].sizes() != t[2].sizes() || t[0].size(1) != t[1].size(1)) Py_RETURN_NONE;
+  if (!at::GradMode::is_enabled() ||
+      !(t[0].requires_grad() || t[1].requires_grad() || t[2].requires_grad())) {
+    // no backward: two of the three [M, H] outputs are not written
+    const c10::DeviceGuard guard(dev);
+    const at::NoGradGuard no_grad;
+    Tensor a, b;
+    return THPVariable_Wrap(
+        gate_up_forward(rows_bf16(t[0]), rows_bf16(t[1]), rows_bf16(t[2]), false, a, b));
+  }
   return THPVariable_Wrap(GateUp::apply(t[0], t[1], t[2]));
   END_HANDLE_TH_ERRORS
 }

@@ -3,17 +3,32 @@
 // in one MFMA kernel (the reference's SwiGLUMLP runs two GEMMs that write a
 // and b to HBM and a SwiGLU kernel that reads them back, model/dit.py:96-110).
 //
-// Tiling.  A 256 x 256 block tile of the combined product x [W_gate; W_up]^T
-// covers 256 tokens and 128 hidden units: tile columns 64 q .. 64 q + 31 are
-// gate units u0 + 32 q .. + 31 and columns 64 q + 32 .. 64 q + 63 the up
-// projections of the same units (u0 = 128 * tile column).  The direct-to-LDS
-// loader hands each wavefront 32 consecutive tile rows of the B operand, so
-// wavefront w simply copies its rows from W_up (w odd) or W_gate (w even):
-// the interleave costs nothing and the weights are used in place.  With 8
-// wavefronts of 128 x 64, a lane's two 32-column accumulator tiles are then
-// a and b of the same (token, unit) pairs, and the epilogue is element-wise
-// in registers: fp32 silu(a) * b rounded once, plus a and b rounded to the
-// input type (what the backward needs; the caller may skip them).
+// Tiling.  A 256 x 256 block tile covers 256 tokens and 128 hidden units: on
+// the weights' side, tile rows 64 q .. 64 q + 31 are gate units u0 + 32 q .. + 31
+// and rows 64 q + 32 .. 64 q + 63 the up projections of the same units (u0 =
+// 128 * the tile's index along H).  The direct-to-LDS loader hands each
+// wavefront 32 consecutive tile rows of an operand, so wavefront w simply
+// copies its rows from W_up (w odd) or W_gate (w even): the interleave costs
+// nothing and the weights are used in place.  A lane's accumulator tiles are
+// then a and b of the same (token, unit) pairs, and the epilogue is
+// element-wise in registers: fp32 silu(a) * b rounded once, plus a and b
+// rounded to the input type (what the backward needs; the caller may skip
+// them).
+//
+// With the weights as the A operand (VEC) a lane holds 4 consecutive units of a
+// token's row per tile quarter, and one exchange between the lane halves makes
+// 16-byte stores, 8 a lane and output; with the tokens as A the values go out
+// two bytes at a time, 64 stores a lane and output, each 64 contiguous bytes of
+// two rows.  Tokens as A -> weights as A, us:
+//   act alone:  M 9408 D 384 H 1536 32.5 -> 29.4, M 4096 D 2048 H 5632 153 -> 150,
+//               M 2392 D 728 H 5392 49.5 -> 46.3, M 2048 D 384 H 1536 15.4 -> 13.8,
+//               M 64 D 256 H 512 11.7 -> 10.1
+//   a, b, act:  38.9 -> 40.4, 161 -> 164, 54.3 -> 56.5, 18.1 -> 18.9, 12.9 -> 11.5
+// act alone is bound by the number of stores, three outputs by their traffic,
+// where the longer contiguous pieces do better (64 bytes a row by one more
+// exchange, or an output after the other so that a row's 128-byte line fills in
+// four stores, changed nothing).  So VEC takes the call that wants act alone,
+// and three outputs keep the tokens as A.
 #include "gemm_store.h"
 
 namespace nf {
@@ -23,7 +38,8 @@ using C = gemm::DCfg<256, 256, 2, 4, 2, 64>;
 using gemm::floatx16;
 static_assert(C::BN == 256 && C::NW == 8 && C::WM == 2 && C::WN == 4, "tiling assumed below");
 static_assert(C::BCW * C::RPC == 32, "each wavefront must copy one 32-row group of B");
-static_assert(C::TN == 2, "a lane's two column tiles are the gate and up halves");
+static_assert(C::ACW == C::BCW, "the weights take either side of the product");
+static_assert(C::TN == 2 && C::TM == 4, "a lane's tiles pair up as gate and up halves");
 
 constexpr uint32_t kOob = 0x80000000u;
 
@@ -47,7 +63,36 @@ __device__ __forceinline__ void st_bf16(__amdgpu_buffer_rsrc_t r, uint32_t off, 
   __builtin_amdgcn_raw_buffer_store_b16(bits, r, ok ? off : kOob, 0, 0);
 }
 
-template <bool BUF>
+// A lane's 16 values of one 32 x 32 tile (units 8 g + 4 half .. + 3 of its
+// token's row, g = 0..3) as two 16-byte stores: the swap of quarters g and
+// g + 1 between the lane halves leaves lanes 0-31 with all 8 units of g, lanes
+// 32-63 with those of g + 1.  The tile's first unit is the u0-th from byte
+// offset `off`, and the row has `units` from there.
+__device__ __forceinline__ void st_row32(__amdgpu_buffer_rsrc_t rs, uint32_t off, int u0,
+                                         int units, const float (&v)[16]) {
+  const int half = (threadIdx.x & 63) >> 5;
+#pragma unroll
+  for (int g = 0; g < 4; g += 2) {
+    uint32_t a[2], b[2];
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+      const int lo = 4 * g + 2 * q, hi = lo + 4;
+      a[q] = (uint32_t)gemm::to_half_bits(v[lo], NF_DTYPE_BF16) |
+             ((uint32_t)gemm::to_half_bits(v[lo + 1], NF_DTYPE_BF16) << 16);
+      b[q] = (uint32_t)gemm::to_half_bits(v[hi], NF_DTYPE_BF16) |
+             ((uint32_t)gemm::to_half_bits(v[hi + 1], NF_DTYPE_BF16) << 16);
+    }
+    const auto s0 = __builtin_amdgcn_permlane32_swap(a[0], b[0], false, false);
+    const auto s1 = __builtin_amdgcn_permlane32_swap(a[1], b[1], false, false);
+    const u32x4 pk = {s0[0], s1[0], s0[1], s1[1]};
+    const int u = u0 + 8 * (g + half);
+    __builtin_amdgcn_raw_buffer_store_b128(pk, rs, u < units ? off + 2 * u : kOob, 0, 0);
+  }
+}
+
+// VEC: act alone, in rows of whole 16-byte vectors, the weights as the A
+// operand (see the top).
+template <bool BUF, bool VEC>
 __global__ NF_GEMM_BOUNDS(C) void gate_up_swiglu_kernel(Args p) {
   __shared__ __attribute__((aligned(16))) char smem[C::LDS_BYTES];
   int tm, tn;
@@ -64,41 +109,62 @@ __global__ NF_GEMM_BOUNDS(C) void gate_up_swiglu_kernel(Args p) {
     for (int j = 0; j < C::TN; ++j)
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
-  gemm::DtlOperand<C, C::ACW> opa;
-  gemm::DtlOperand<C, C::BCW> opb;
-  opa.init(p.x, p.ldx, p.M, p.D, m0, wave);
+  gemm::DtlOperand<C, C::ACW> opx;
+  gemm::DtlOperand<C, C::BCW> opw;
+  opx.init(p.x, p.ldx, p.M, p.D, m0, wave);
   // wavefront w copies tile rows 32 w .. 32 w + 31: units u0 + 32 (w / 2) + 0..31
   // of W_up (w odd) or W_gate (w even); r0 makes tile row 32 w that matrix row
   const int64_t unit0 = u0 + 32 * (wave >> 1);
-  opb.init((wave & 1) ? p.wu : p.wg, (wave & 1) ? p.ldu : p.ldg, p.H, p.D, unit0 - 32 * wave,
+  opw.init((wave & 1) ? p.wu : p.wg, (wave & 1) ? p.ldu : p.ldg, p.H, p.D, unit0 - 32 * wave,
            wave);
-  gemm::mainloop_dtl_ops<C, BUF, true>(opa, opb, p.D, smem, acc);
+  if constexpr (VEC)
+    gemm::mainloop_dtl_ops<C, BUF, true>(opw, opx, p.D, smem, acc);
+  else
+    gemm::mainloop_dtl_ops<C, BUF, true>(opx, opw, p.D, smem, acc);
 
   const int l = threadIdx.x & 63;
   const int w = threadIdx.x >> 6, wm = w / C::WN, wn = w % C::WN;
-  const int64_t unit = u0 + 32 * wn + (l & 31);
-  const int64_t row0 = m0 + wm * C::WTM + 4 * (l >> 5);
   const int64_t bytes = p.M * p.ldo * 2;
   const __amdgpu_buffer_rsrc_t ract =
       __builtin_amdgcn_make_buffer_rsrc(p.act, (short)0, (int)bytes, 0x00020000);
-  __amdgpu_buffer_rsrc_t ra = ract, rb = ract;
-  if (p.a) ra = __builtin_amdgcn_make_buffer_rsrc(p.a, (short)0, (int)bytes, 0x00020000);
-  if (p.b) rb = __builtin_amdgcn_make_buffer_rsrc(p.b, (short)0, (int)bytes, 0x00020000);
-  const bool save = p.a != nullptr;
+  if constexpr (VEC) {
 #pragma unroll
-  for (int i = 0; i < C::TM; ++i)
-#pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      const int64_t row = row0 + i * 32 + 8 * (r >> 2) + (r & 3);
-      const bool ok = row < p.M && unit < p.H;
+    for (int j = 0; j < C::TN; ++j) {
+      const int64_t row = m0 + wn * C::WTN + j * 32 + (l & 31);
+      const int64_t unit = u0 + 32 * (wm * (C::TM / 2));
       const uint32_t off = (uint32_t)((row * p.ldo + unit) * 2);
-      const float av = acc[i][0][r], bv = acc[i][1][r];
-      st_bf16(ract, off, ok, av * sigmoid(av) * bv);
-      if (save) {
-        st_bf16(ra, off, ok, av);
-        st_bf16(rb, off, ok, bv);
+      const int units = row < p.M ? (int)(p.H - unit < 64 ? p.H - unit : 64) : 0;  // <= 0: none
+#pragma unroll
+      for (int i = 0; i < C::TM; i += 2) {  // tiles i, i + 1: gate and up of 32 units
+        float v[16];
+#pragma unroll
+        for (int r = 0; r < 16; ++r)
+          v[r] = acc[i][j][r] * sigmoid(acc[i][j][r]) * acc[i + 1][j][r];
+        st_row32(ract, off, 16 * i, units, v);
       }
     }
+  } else {
+    __amdgpu_buffer_rsrc_t ra = ract, rb = ract;
+    if (p.a) ra = __builtin_amdgcn_make_buffer_rsrc(p.a, (short)0, (int)bytes, 0x00020000);
+    if (p.b) rb = __builtin_amdgcn_make_buffer_rsrc(p.b, (short)0, (int)bytes, 0x00020000);
+    const bool save = p.a != nullptr;
+    const int64_t unit = u0 + 32 * wn + (l & 31);
+    const int64_t row0 = m0 + wm * C::WTM + 4 * (l >> 5);
+#pragma unroll
+    for (int i = 0; i < C::TM; ++i)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const int64_t row = row0 + i * 32 + 8 * (r >> 2) + (r & 3);
+        const bool ok = row < p.M && unit < p.H;
+        const uint32_t off = (uint32_t)((row * p.ldo + unit) * 2);
+        const float av = acc[i][0][r], bv = acc[i][1][r];
+        st_bf16(ract, off, ok, av * sigmoid(av) * bv);
+        if (save) {
+          st_bf16(ra, off, ok, av);
+          st_bf16(rb, off, ok, bv);
+        }
+      }
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -185,10 +251,14 @@ extern "C" int nf_gemm_swiglu(const void *x, int64_t ldx, const void *w_gate, in
                    aligned16(x) && aligned16(w_gate) && aligned16(w_up);
   hipStream_t s = static_cast<hipStream_t>(stream);
   const unsigned grid = (unsigned)(tiles_m * tiles_n);
-  if (buf)
-    gate_up_swiglu_kernel<true><<<grid, C::NT, 0, s>>>(args);
+  // 16-byte stores where they are possible and win (measured at the top)
+  const bool vec = buf && !a && H % 8 == 0 && ldo % 8 == 0 && aligned16(act);
+  if (vec)
+    gate_up_swiglu_kernel<true, true><<<grid, C::NT, 0, s>>>(args);
+  else if (buf)
+    gate_up_swiglu_kernel<true, false><<<grid, C::NT, 0, s>>>(args);
   else
-    gate_up_swiglu_kernel<false><<<grid, C::NT, 0, s>>>(args);
+    gate_up_swiglu_kernel<false, false><<<grid, C::NT, 0, s>>>(args);
   return check_launch("nf_gemm_swiglu");
 }
 

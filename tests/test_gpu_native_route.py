@@ -113,6 +113,30 @@ def test_gate_up_route_matches_the_function(cuda, xd, gd, ud, need):
               _grads(swiglu._FusedGateUpSwiGLU.apply, [x, wg, wu], need, up))
 
 
+@pytest.mark.parametrize("m,d,h", [(300, 136, 264), (5, 64, 1000), (300, 36, 100)])
+@pytest.mark.parametrize("dtype", [BF16, F32])
+def test_gate_up_without_a_backward(cuda, m, d, h, dtype):
+    """No backward to come (no_grad, or no input that wants a gradient): only
+    act is written; the forward of a training step is the reference, one bf16
+    rounding (an ulp, 2^-7, at most) apart."""
+    note(f"native gate/up inference m={m} d={d} h={h} {dtype}")
+    g = gen(8)
+    x = randn((m, d), g, dtype, cuda)
+    w = [randn((h, d), g, dtype, cuda, std=d ** -0.5).requires_grad_(True) for _ in range(2)]
+    with torch.autocast("cuda", dtype=BF16):
+        want = fused_gate_up_swiglu(x, *w)
+        assert want.requires_grad
+        with torch.no_grad():
+            got = [fused_gate_up_swiglu(x, *w)]
+        with torch.inference_mode():
+            got.append(fused_gate_up_swiglu(x, *w))
+        got.append(fused_gate_up_swiglu(x, *(v.detach() for v in w)))
+    ref = want.detach().float()
+    for act in got:
+        assert act.dtype == BF16 and act.shape == (m, h) and not act.requires_grad
+        assert ((act.float() - ref).abs() <= 2.0 ** -7 * ref.abs() + 1e-5).all()
+
+
 def test_saved_tensors_go_through_the_hooks(cuda):
     note("native route under saved-tensor hooks")
     inputs, up, t = _seam_inputs(cuda, F32, BF16)

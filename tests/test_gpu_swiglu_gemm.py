@@ -19,6 +19,7 @@ import pytest
 import torch
 import torch.nn.functional as F
 
+from nuvla_forge_amd import _lib
 from nuvla_forge_amd.kernels import fused_gate_up_swiglu
 from oracle import numerics as on
 from tests.helpers import gen, note, np64, randn
@@ -62,6 +63,41 @@ def test_gate_up_swiglu_matches_oracle(cuda, m, d, h):
     errs = {k: on.rel_err(np64(v), r)
             for k, v, r in zip(("act", "dx", "dwg", "dwu"), (act, dx, dwg, dwu), ref)}
     assert all(e <= 2e-2 for e in errs.values()), errs
+
+
+# act alone takes the epilogue with 16-byte stores: tile edges (256 tokens, 128
+# units), remainders of the 32-unit groups, output rows wider than H; beside it
+# the same product with rows one element longer, which are not whole vectors
+# and go out element by element, as a, b and act together do
+@pytest.mark.parametrize("m,d,h,pad", [(256, 64, 128, 0), (257, 72, 136, 8), (255, 136, 24, 0),
+                                       (31, 8, 8, 16), (513, 200, 264, 0), (1, 64, 1000, 8)])
+@pytest.mark.parametrize("save", [True, False])
+def test_gate_up_entry_rows_of_whole_vectors(cuda, m, d, h, pad, save):
+    note(f"gate/up entry m={m} d={d} h={h} pad={pad} save={save}")
+    x, wg, wu, _ = _inputs(m, d, h, torch.bfloat16, cuda, seed=m + h)
+    L = _lib.lib()
+
+    def run(ldo):
+        outs = [torch.full((m, ldo), -7.0, dtype=torch.bfloat16, device=cuda)
+                for _ in range(3 if save else 1)]
+        ab = [o.data_ptr() for o in outs[1:]] if save else [None, None]
+        _lib.check(L.nf_gemm_swiglu(x.data_ptr(), d, wg.data_ptr(), d, wu.data_ptr(), d, *ab,
+                                    outs[0].data_ptr(), ldo, m, d, h,
+                                    _lib.dtype_code(torch.bfloat16), _lib.stream_of(x)),
+                   "nf_gemm_swiglu")
+        torch.cuda.synchronize()
+        for o in outs:
+            assert (o[:, h:] == -7.0).all()  # nothing past a row's H
+        return [np64(o[:, :h]) for o in outs]
+
+    a, b = np64(x) @ np64(wg).T, np64(x) @ np64(wu).T
+    want = [on.swiglu_forward(a, b), a, b]
+    # each result is rounded to bf16 once: 2^-8 of it at most (8 significant
+    # bits).  A sum of up to 200 products rounds ~13 times to 2^-24 of at most
+    # sum |x w| ~ 10, 1e-5 absolute; silu(a) b carries that times |a|, |b| < 6.
+    for got in (run(h + pad), run(h + pad + 1)):
+        for g, w in zip(got, want):
+            assert (np.abs(g - w) <= 2.0 ** -8 * np.abs(w) + 6e-5).all()
 
 
 def test_gate_up_swiglu_weights_with_different_row_strides(cuda):
