@@ -9,7 +9,7 @@ ignore_index=-100, force_reference=False)`` (chunked_ce.py:185-208).
 
 The device path is two calls.  ``nf_ce_fwd`` compacts the valid rows on the
 device and, ``chunk_size`` of them at a time, forms their logits once on
-bf16 (or fp32) MFMA and keeps them as ``exp(logit - target logit)`` in both
+bf16 MFMA (fp32 values as three bf16 parts) and keeps them as ``exp(logit - target logit)`` in both
 layouts the gradient products read, with a per-row factor (from an fp32
 log-sum-exp over per-tile statistics) that makes them ``(softmax - onehot) /
 n``; it runs the gradient products of every chunk but the last, and the loss
@@ -42,7 +42,8 @@ on chunk_size beyond fp rounding.
 Element types: under bf16 autocast for the device the products run in bf16
 (MFMA, fp32 accumulation) whatever the input types, as the reference's
 autocast-ed ``F.linear`` and ``@`` do; otherwise bf16 inputs run bf16 MFMA,
-fp32 inputs fp32 MFMA, and mixed or fp16 inputs are widened to fp32.
+fp32 inputs six bf16 products over three-part operands (more precise than fp32
+MFMA), and mixed or fp16 inputs are widened to fp32.
 """
 
 from __future__ import annotations
