@@ -786,7 +786,9 @@ __device__ __forceinline__ void split8(const u32x4 (&x)[2], u32x4 (&part)[3]) {
   for (int p = 0; p < 4; ++p) {  // pairs
     const uint32_t u0 = x[p >> 1][2 * (p & 1)], u1 = x[p >> 1][2 * (p & 1) + 1];
     const float f0 = __uint_as_float(u0), f1 = __uint_as_float(u1);
-    const uint32_t h0 = u0 & 0xffff0000u, h1 = u1 & 0xffff0000u;
+    // quieted first: a NaN with payload in its low bits only would be cut to an infinity
+    const uint32_t h0 = __float_as_uint(__builtin_canonicalizef(f0)) & 0xffff0000u;
+    const uint32_t h1 = __float_as_uint(__builtin_canonicalizef(f1)) & 0xffff0000u;
     // an infinity is its own first part, with nothing left
     const float r0 = (u0 & 0x7fffffffu) == 0x7f800000u ? 0.f : f0 - __uint_as_float(h0);
     const float r1 = (u1 & 0x7fffffffu) == 0x7f800000u ? 0.f : f1 - __uint_as_float(h1);

@@ -69,3 +69,16 @@ def test_split_gemm_keeps_infinities_and_nan(cuda):
     got = _gemm(a, b, 32).cpu()
     assert (got[0] == inf).all() and (got[1] == -inf).all() and got[2].isnan().all()
     assert (got[3] == 16.0).all()
+
+
+# signalling NaNs, positive and negative, whose payload lies in the 16 bits
+# below the first part
+@pytest.mark.parametrize("bits", [0x7f800001, 0x7f80ffff, 0xff800001 - (1 << 32)])
+def test_split_gemm_keeps_nan_payloads_nan(cuda, bits):
+    note(f"split gemm: nan bits {bits:#x}")
+    a = torch.ones(3, 32, device=cuda)
+    a.view(torch.int32)[1, 7] = bits
+    b = torch.full((2, 32), 0.5, device=cuda)
+    got = _gemm(a, b, 32).cpu()
+    assert got[1].isnan().all()
+    assert (got[0] == 16.0).all() and (got[2] == 16.0).all()
