@@ -17,6 +17,7 @@
 #include <torch/csrc/autograd/custom_function.h>
 #include <torch/csrc/autograd/python_variable.h>
 #include <torch/csrc/jit/frontend/tracer.h>
+#include <torch/csrc/utils/pybind.h>
 #include <torch/torch.h>
 #include <ATen/PythonTorchFunctionTLS.h>
 #include <c10/core/DeviceGuard.h>
@@ -331,6 +332,15 @@ bool tensors(PyObject *const *args, Py_ssize_t nargs, Py_ssize_t want, Tensor (&
   return true;
 }
 
+// The call without the interpreter lock, which other threads take meanwhile (an
+// allocation or a launch may wait); what calls into Python, such as a
+// saved-tensor hook, takes it for itself.
+template <class F>
+auto unlocked(F &&f) {
+  const pybind11::gil_scoped_release no_gil;
+  return f();
+}
+
 PyObject *py_seam(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
   HANDLE_TH_ERRORS
   Tensor a[6];
@@ -342,7 +352,8 @@ PyObject *py_seam(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
     Py_RETURN_NONE;
   }
   if (!seam_plain(a[0], a[1], a[2], a[3], a[4], a[5], t)) Py_RETURN_NONE;
-  const variable_list r = Seam::apply(a[0], a[1], a[2], a[3], a[4], a[5], t, eps);
+  const variable_list r =
+      unlocked([&] { return Seam::apply(a[0], a[1], a[2], a[3], a[4], a[5], t, eps); });
   PyObject *h = THPVariable_Wrap(r[0]), *out = THPVariable_Wrap(r[1]);
   PyObject *pair = PyTuple_Pack(2, h, out);
   Py_XDECREF(h);
@@ -359,7 +370,7 @@ PyObject *py_swiglu(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
   if (!plain(t[0], dev) || !plain(t[1], dev) || t[0].sizes() != t[1].sizes() ||
       t[0].scalar_type() != t[1].scalar_type() || code_of(t[0]) < 0 || t[0].numel() == 0)
     Py_RETURN_NONE;
-  return THPVariable_Wrap(SwiGLU::apply(t[0], t[1]));
+  return THPVariable_Wrap(unlocked([&] { return SwiGLU::apply(t[0], t[1]); }));
   END_HANDLE_TH_ERRORS
 }
 
@@ -375,13 +386,14 @@ PyObject *py_gate_up(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
   if (!at::GradMode::is_enabled() ||
       !(t[0].requires_grad() || t[1].requires_grad() || t[2].requires_grad())) {
     // no backward: two of the three [M, H] outputs are not written
-    const c10::DeviceGuard guard(dev);
-    const at::NoGradGuard no_grad;
-    Tensor a, b;
-    return THPVariable_Wrap(
-        gate_up_forward(rows_bf16(t[0]), rows_bf16(t[1]), rows_bf16(t[2]), false, a, b));
+    return THPVariable_Wrap(unlocked([&] {
+      const c10::DeviceGuard guard(dev);
+      const at::NoGradGuard no_grad;
+      Tensor a, b;
+      return gate_up_forward(rows_bf16(t[0]), rows_bf16(t[1]), rows_bf16(t[2]), false, a, b);
+    }));
   }
-  return THPVariable_Wrap(GateUp::apply(t[0], t[1], t[2]));
+  return THPVariable_Wrap(unlocked([&] { return GateUp::apply(t[0], t[1], t[2]); }));
   END_HANDLE_TH_ERRORS
 }
 
@@ -405,7 +417,8 @@ PyObject *py_ce(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
       code_of(t[0]) < 0 || code_of(t[1]) < 0 || t[2].scalar_type() != at::kLong || v[0] <= 0)
     Py_RETURN_NONE;
   const at::ScalarType cdt = v[2] == NF_DTYPE_BF16 ? at::kBFloat16 : at::kFloat;
-  return THPVariable_Wrap(ChunkedCE::apply(t[0], t[1], t[2], v[0], v[1], (int64_t)cdt));
+  return THPVariable_Wrap(unlocked(
+      [&] { return ChunkedCE::apply(t[0], t[1], t[2], v[0], v[1], (int64_t)cdt); }));
   END_HANDLE_TH_ERRORS
 }
 

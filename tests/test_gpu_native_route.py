@@ -8,6 +8,8 @@ behaves as the Functions always did.
 
 from __future__ import annotations
 
+from concurrent.futures import ThreadPoolExecutor
+
 import pytest
 import torch
 
@@ -204,3 +206,29 @@ def test_native_route_on_another_stream(cuda):
     torch.cuda.current_stream().wait_stream(side)
     torch.cuda.synchronize()
     _same(got, want)
+
+
+def test_native_route_from_several_threads(cuda):
+    """Four threads, a stream each, take turns at the interpreter while others
+    are inside a call: each gets what a thread of its own gets."""
+    note("native route from four threads")
+    inputs, up, t = _seam_inputs(cuda, BF16, BF16, b=4, t=16, n=512, pad=0)
+
+    def step():
+        return _grads(lambda *v: fused_adaln_residual_rmsnorm(*v, tokens_per_sample=t), inputs,
+                      (True,) * 6, up)
+
+    want = step()
+    torch.cuda.synchronize()
+
+    def work(_):
+        stream = torch.cuda.Stream()
+        with torch.cuda.stream(stream):
+            outs = [step() for _ in range(8)]
+        stream.synchronize()
+        return outs
+
+    with ThreadPoolExecutor(4) as ex:
+        for outs in ex.map(work, range(4)):
+            for got in outs:
+                _same(got, want)
