@@ -404,7 +404,10 @@ PyObject *py_ce(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
   Tensor t[3];
   if (!tensors(args, nargs, 6, t) || !quiet()) Py_RETURN_NONE;
   int64_t v[3];
-  for (int i = 0; i < 3; ++i) v[i] = PyLong_Check(args[3 + i]) ? PyLong_AsLongLong(args[3 + i]) : -1;
+  for (int i = 0; i < 3; ++i) {
+    if (!PyLong_Check(args[3 + i])) Py_RETURN_NONE;  // the general path converts it
+    v[i] = PyLong_AsLongLong(args[3 + i]);
+  }
   if (PyErr_Occurred()) {
     PyErr_Clear();
     Py_RETURN_NONE;

@@ -10,6 +10,7 @@ from __future__ import annotations
 
 from concurrent.futures import ThreadPoolExecutor
 
+import numpy as np
 import pytest
 import torch
 
@@ -99,6 +100,27 @@ def test_ce_route_matches_the_function(cuda, hd, wd, autocast):
         slow = _grads(lambda h, v: chunked_ce._ChunkedCrossEntropy.apply(h, v, tgt, 32, -1, False),
                       [hid, w], (True, True), up)
     _same(fast, slow)
+
+
+@pytest.mark.parametrize("index", [np.int64(7), torch.tensor(7), 7.0])
+def test_ce_ignore_index_that_is_no_python_int(cuda, index):
+    """A class of the vocabulary masked by an index of another type: what the
+    plain int gives, to the bit, and the native entry answers None."""
+    note(f"native ce ignore_index {index!r}")
+    g = gen(9)
+    hid, w = randn((64, 40), g, F32, cuda), randn((50, 40), g, F32, cuda)
+    tgt = torch.randint(0, 50, (64,), generator=g)
+    tgt[::3] = 7
+    tgt = tgt.to(cuda)
+    assert _lib.native().ce(hid, w, tgt, 16, index, 0) is None
+    assert _lib.native().ce(hid, w, tgt, np.int64(16), 7, 0) is None
+    up = [torch.tensor(1.0, device=cuda)]
+    want = _grads(lambda h, v: chunked_cross_entropy(h, v, tgt, 16, 7), [hid, w], (True, True), up)
+    for chunk in (16, np.int64(16)):
+        got = _grads(lambda h, v: chunked_cross_entropy(h, v, tgt, chunk, index), [hid, w],
+                     (True, True), up)
+        _same(got, want)
+    assert (want[1][::3] == 0).all()  # the masked rows have no gradient
 
 
 @pytest.mark.parametrize("xd,gd,ud", [(BF16, BF16, BF16), (F32, F32, F32), (F32, BF16, F32)])
