@@ -247,22 +247,24 @@ struct GateUp : torch::autograd::Function<GateUp> {
     check(nf_swiglu_bwd(dact.data_ptr(), a.data_ptr(), b.data_ptr(), da.data_ptr(),
                         db.data_ptr(), a.numel(), NF_DTYPE_BF16, st),
           "nf_swiglu_bwd");
-    // both weight gradients leave the kernel in one type; they differ only
-    // where the weights do
+    // both weight gradients leave the kernel in one type: theirs, or fp32 where
+    // two are wanted and differ (neither may round the other's gradient)
     const auto tx = (at::ScalarType)dt[0], tg = (at::ScalarType)dt[1], tu = (at::ScalarType)dt[2];
+    const bool need_g = ctx->needs_input_grad(1), need_u = ctx->needs_input_grad(2);
+    const auto tw = need_g && need_u && tg != tu ? at::kFloat : need_g ? tg : tu;
     Tensor dx, dg, du;
     if (ctx->needs_input_grad(0)) dx = at::empty({m, d}, x.options().dtype(tx));
-    if (ctx->needs_input_grad(1)) dg = at::empty({h, d}, x.options().dtype(tg));
-    if (ctx->needs_input_grad(2)) du = at::empty({h, d}, x.options().dtype(tg));
+    if (need_g) dg = at::empty({h, d}, x.options().dtype(tw));
+    if (need_u) du = at::empty({h, d}, x.options().dtype(tw));
     const size_t nb = nf_gemm_swiglu_bwd_workspace(m, d, h, dx.defined(), dg.defined(),
                                                    du.defined());
     Tensor ws = bytes(nb, x);
     check(nf_gemm_swiglu_bwd(da.data_ptr(), db.data_ptr(), h, x.data_ptr(), x.stride(0),
                              wg.data_ptr(), wg.stride(0), wu.data_ptr(), wu.stride(0), ptr(dx),
-                             code_of(tx), ptr(dg), ptr(du), code_of(tg), m, d, h, NF_DTYPE_BF16,
+                             code_of(tx), ptr(dg), ptr(du), code_of(tw), m, d, h, NF_DTYPE_BF16,
                              ws.data_ptr(), nb, st),
           "nf_gemm_swiglu_bwd");
-    return {dx, dg, du.defined() ? du.to(tu) : du};
+    return {dx, need_g ? dg.to(tg) : dg, need_u ? du.to(tu) : du};
   }
 };
 

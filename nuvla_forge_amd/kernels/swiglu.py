@@ -116,25 +116,34 @@ class _FusedGateUpSwiGLU(torch.autograd.Function):
         need = ctx.needs_input_grad
         m, d = x.shape
         h = a.shape[1]
+        # the kernel writes fp32, bf16 or fp16: dx in x's type, both weight
+        # gradients in one, theirs or fp32 where two are wanted and differ
+        # (neither may round the other's gradient); any other type is cast to
+        # from fp32
+        need_x, need_g, need_u = need[:3]
         tx, tg, tu = ctx.dtypes
-        dx = torch.empty((m, d), dtype=tx, device=x.device) if need[0] else None
-        # both weight gradients leave the kernel in one type
-        dwg = torch.empty((h, d), dtype=tg, device=x.device) if need[1] else None
-        dwu = torch.empty((h, d), dtype=tg, device=x.device) if need[2] else None
+        cx = tx if tx in _lib.DTYPE_CODE else torch.float32
+        cw = tg if need_g else tu
+        if (need_g and need_u and tg != tu) or cw not in _lib.DTYPE_CODE:
+            cw = torch.float32
+        dx = torch.empty((m, d), dtype=cx, device=x.device) if need_x else None
+        dwg = torch.empty((h, d), dtype=cw, device=x.device) if need_g else None
+        dwu = torch.empty((h, d), dtype=cw, device=x.device) if need_u else None
         with device_of(x):
-            nbytes = L.nf_gemm_swiglu_bwd_workspace(m, d, h, need[0], need[1], need[2])
+            nbytes = L.nf_gemm_swiglu_bwd_workspace(m, d, h, need_x, need_g, need_u)
             ws = torch.empty(max(nbytes, 1), dtype=torch.uint8, device=x.device)
             _lib.check(
                 L.nf_gemm_swiglu_bwd(da.data_ptr(), db.data_ptr(), h, x.data_ptr(),
                                      x.stride(0), w_gate.data_ptr(), w_gate.stride(0),
                                      w_up.data_ptr(), w_up.stride(0), _lib.ptr(dx),
-                                     _lib.dtype_code(tx), _lib.ptr(dwg), _lib.ptr(dwu),
-                                     _lib.dtype_code(tg), m, d, h,
+                                     _lib.dtype_code(cx), _lib.ptr(dwg), _lib.ptr(dwu),
+                                     _lib.dtype_code(cw), m, d, h,
                                      _lib.dtype_code(torch.bfloat16), ws.data_ptr(), nbytes,
                                      _lib.stream_of(x)),
                 "nf_gemm_swiglu_bwd",
             )
-        return dx, dwg, dwu if dwu is None else dwu.to(tu)
+        return (dx.to(tx) if need_x else None, dwg.to(tg) if need_g else None,
+                dwu.to(tu) if need_u else None)
 
 
 def _gate_up_eager(x, w_gate, w_up):

@@ -137,6 +137,29 @@ def test_gate_up_route_matches_the_function(cuda, xd, gd, ud, need):
               _grads(swiglu._FusedGateUpSwiGLU.apply, [x, wg, wu], need, up))
 
 
+@pytest.mark.parametrize("xd,gd,ud", [
+    (torch.float64,) * 3, (torch.int64, F32, F32), (F32, torch.float64, F32), (F32, F16, F32),
+    (F32, F16, BF16), (BF16, F32, F16), (F16, F16, F16), (F32, BF16, F32)])
+@pytest.mark.parametrize("need", [(True, True, True), (False, True, False), (False, False, True)])
+def test_gate_up_gradients_in_any_input_types(cuda, xd, gd, ud, need):
+    """Each gradient is the fp32 one rounded once to its own input's type: of
+    no other input's type (an fp16 weight beside a bf16 or fp32 one must not
+    overflow the other's gradient), and in types no kernel writes."""
+    note(f"gate/up gradient types {xd}/{gd}/{ud} need={need}")
+    g = gen(10)
+    x = torch.randint(-8, 9, (70, 72), generator=g).to(cuda)  # whole in every type
+    w = [torch.randint(-16, 17, (48, 72), generator=g).to(cuda) / 64 for _ in range(2)]
+    need = (need[0] and xd.is_floating_point, *need[1:])
+    # beyond fp16's range in the weight gradients
+    up = [randn((70, 48), g, BF16, cuda, std=1e4)]
+    with torch.autocast("cuda", dtype=BF16):
+        want = _grads(fused_gate_up_swiglu, [x.float(), *w], need, up)
+        got = _grads(fused_gate_up_swiglu, [x.to(xd), w[0].to(gd), w[1].to(ud)], need, up)
+    types = [BF16, *(t for t, k in zip((xd, gd, ud), need) if k)]
+    assert max(v.abs().max() for v in want[1:]) > torch.finfo(F16).max
+    _same(got, [v.to(t) for v, t in zip(want, types)])
+
+
 @pytest.mark.parametrize("m,d,h", [(300, 136, 264), (5, 64, 1000), (300, 36, 100)])
 @pytest.mark.parametrize("dtype", [BF16, F32])
 def test_gate_up_without_a_backward(cuda, m, d, h, dtype):
