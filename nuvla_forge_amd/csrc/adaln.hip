@@ -427,7 +427,9 @@ extern "C" int nf_adaln_bwd_full(const void *dh_up, const void *dout, const void
   if (!is_dtype(dt_gate) || !is_dtype(dt_weight) || !is_dtype(dt_scale) || !is_dtype(dt_shift))
     return set_error(NF_ERR_DTYPE, "nf_adaln_bwd_full: bad conditioning dtype");
   const Plan pl = M > 0 ? make_plan(M, N, T) : Plan{};
-  const WalkPlan w = M > 0 ? make_walk_plan(pl, N, T) : WalkPlan{};
+  const int64_t bytes16 = dt_x == NF_DTYPE_F32 ? 0
+      : M * ((N + 511) / 512 * 512) * 2 * (2 + (dh_up ? 1 : 0) + (dout ? 1 : 0));
+  const WalkPlan w = M > 0 ? make_walk_plan(pl, N, T, bytes16) : WalkPlan{};
   const bool any = dgate || dweight || dscale || dshift;
   if (w.use && any && x && y && gate && weight && scale && rstd && dx && dy && workspace &&
       workspace_bytes_given >= workspace_bytes(pl, N) && ld_x >= N && ld_y >= N &&

@@ -1061,24 +1061,62 @@ struct WalkPlan {
 // It runs when the plan would give every sample a block of its own and more
 // than one round of them (B above the blocks aimed at); with fewer samples
 // the blocks of adaln_bwd_kernel are all resident and the reduction takes at
-// most 8 rounds.  A row group walks samples alone when that makes at least
-// kWalkGroupWaves wavefronts (8 per CU), or when the sample has fewer rows
-// than a block has groups; otherwise the block's groups share each sample.
+// most 8 rounds.  One chunk per lane only (N <= 4096): with two its two row
+// buffers spill 200-470 registers, and the row kernel and reduction win: x fp32,
+// y bf16, forward + backward, [257, 33, 4104] 345 us against 757, bf16
+// [600, 33, 6144] 634 against 1026.
+// 177-210 VGPRs hold two wavefronts a SIMD, so kWalkSlots blocks of 256 threads
+// run at once, or half as many of 512.  A row group walks samples alone when
+// that makes at least kWalkGroupWaves wavefronts (8 per CU), or when the sample
+// has fewer rows than a block has groups; otherwise, and for long samples where
+// that makes fewer rounds, the block's groups share each sample.  Blocks past
+// kWalkMaxBlocks take more samples each, unless one sample fewer a unit makes
+// fewer rounds of long samples: bf16 forward + backward [1030, 323, 256] 525 ->
+// 440 us, [1250, 44, 1536] 410 -> 341 (short ones lose 2-4 us to the dweight
+// rows).
+// `bytes16`: what the pipelined row kernel would stream in (whole wavefronts),
+// 0 where it does not take the types.  It streams 10-20% faster, so beyond the
+// caches, where its partial rows weigh little, it keeps the sample counts that
+// leave the walk's second round half empty (513 to 768; with more samples the
+// reduction's 1.7 us per 32 is the longer): bf16 forward + backward [600, 341, 384]
+// 334 us against 356, [600, 853, 256] 619 against 746; below kWalkRowBytes the
+// walk is level or ahead ([600, 42, 3072] 327 against 369).  So it does the
+// fewest samples of rows that leave half a wavefront's lanes idle ([257, 1294,
+// 256] 491 against 532; [512, 600, 256] 338 against 330).
 constexpr int kWalkGroupWaves = 2048;
 constexpr int kWalkMaxBlocks = 1024;  // also the dweight rows to be added
-inline WalkPlan make_walk_plan(const Plan &pl, int64_t N, int64_t T) {
+constexpr int kWalkSlots = 512;
+constexpr int64_t kWalkRowBytes = (int64_t)600 << 20;
+inline WalkPlan make_walk_plan(const Plan &pl, int64_t N, int64_t T, int64_t bytes16) {
   WalkPlan w{};
-  w.use = pl.B > kBwdBlocksTarget && T <= INT32_MAX / 64 && N % 8 == 0 &&
-          (pl.bwd_k == 1 ? pl.bwd_wpr <= 8 : pl.bwd_wpr == 8);
+  w.use = pl.B > kBwdBlocksTarget && T <= INT32_MAX / 64 && N % 8 == 0 && pl.bwd_k == 1;
   if (!w.use) return w;
   const int R = 64 * pl.bwd_wpr;
   const int G = (R < kWalkMinBlock ? kWalkMinBlock : R) / R;
-  w.coop = G > 1 && T >= G && pl.B * pl.bwd_wpr < kWalkGroupWaves;
-  const int64_t per_block = w.coop ? 1 : G;  // units per block
-  int64_t pu = (pl.B + per_block * kWalkMaxBlocks - 1) / (per_block * kWalkMaxBlocks);
-  w.per_unit = (int)pu;
-  const int64_t units = (pl.B + pu - 1) / pu;
-  w.blocks = (unsigned)((units + per_block - 1) / per_block);
+  const int slots = R > kWalkMinBlock ? kWalkSlots / 2 : kWalkSlots;
+  const bool long_samples = T >= 8 * G;
+  // units of pu samples, per_block of them a block: blocks, and the samples a
+  // slot takes in turn
+  auto blocks = [&](int64_t pu, int64_t per_block) {
+    return ((pl.B + pu - 1) / pu + per_block - 1) / per_block;
+  };
+  auto turns = [&](int64_t pu, int64_t per_block) {
+    return (blocks(pu, per_block) + slots - 1) / slots * pu * per_block;
+  };
+  auto pick = [&](int64_t per_block) {
+    const int64_t pu = (pl.B + per_block * kWalkMaxBlocks - 1) / (per_block * kWalkMaxBlocks);
+    const bool fewer = long_samples && pu > 1 && turns(pu - 1, per_block) < turns(pu, per_block);
+    return fewer ? pu - 1 : pu;
+  };
+  w.coop = G > 1 && T >= G &&
+           (pl.B * pl.bwd_wpr < kWalkGroupWaves ||
+            (long_samples && turns(pick(1), 1) < turns(pick(G), G)));
+  const int64_t per_block = w.coop ? 1 : G;
+  w.per_unit = (int)pick(per_block);
+  w.blocks = (unsigned)blocks(w.per_unit, per_block);
+  if (bytes16 > kWalkRowBytes && pl.B <= 3 * kBwdBlocksTarget && slots == kWalkSlots &&
+      (w.blocks > slots || (N <= 256 && 4 * pl.B < 3 * slots)))
+    w.use = false;
   return w;
 }
 
@@ -1141,14 +1179,17 @@ template <typename TX, typename TY, int K>
 constexpr bool bwd_pipelined() {
   return sizeof(TX) == 2 && sizeof(TY) == 2 && K == 1;
 }
+// Bytes the backward streams in per element of the [M, N] activations.
+template <typename TX, typename TY>
+int64_t bwd_row_bytes(const BwdArgs &a) {
+  return (int64_t)(sizeof(TX) * (1 + (a.dout ? 1 : 0) + (a.dh_up ? 1 : 0)) + sizeof(TY));
+}
 template <typename TX, typename TY, bool VEC, int WPR, int K>
 int launch_bwd_t(const BwdArgs &a, const Plan &pl, hipStream_t s) {
   using S = BwdShape<WPR>;
   const unsigned grid = (unsigned)(pl.B * a.J);
   if constexpr (VEC && bwd_pipelined<TX, TY, K>()) {
-    const int64_t in_row = (int64_t)(sizeof(TX) * (1 + (a.dout ? 1 : 0) + (a.dh_up ? 1 : 0)) +
-                                     sizeof(TY));
-    const bool ntl = nt_loads_for(a.M * a.N * in_row);
+    const bool ntl = nt_loads_for(a.M * a.N * bwd_row_bytes<TX, TY>(a));
     if (pl.bwd_rb == 2 && ntl)
       adaln_bwd_pipe_kernel<TX, TY, K, WPR, kBwdNT, 2, true><<<grid, S::BLK, 0, s>>>(a);
     else if (pl.bwd_rb == 2)
@@ -1168,14 +1209,25 @@ int launch_bwd_t(const BwdArgs &a, const Plan &pl, hipStream_t s) {
   return check_launch("nf_adaln_bwd");
 }
 
-template <typename TX, typename TY, int WPR, int K>
-int launch_walk_t(const BwdArgs &a, const WalkOut &o, const WalkPlan &w, hipStream_t s) {
-  constexpr int BLK = BwdShape<WPR, kWalkMinBlock>::BLK;
-  if (w.coop)
-    adaln_bwd_walk_kernel<TX, TY, K, WPR, true, kBwdNT, false><<<w.blocks, BLK, 0, s>>>(a, o);
-  else
-    adaln_bwd_walk_kernel<TX, TY, K, WPR, false, kBwdNT, false><<<w.blocks, BLK, 0, s>>>(a, o);
+template <typename TX, typename TY, int WPR, bool NTL>
+int launch_walk_c(const BwdArgs &a, const WalkOut &o, const WalkPlan &w, hipStream_t s) {
+  using S = BwdShape<WPR, kWalkMinBlock>;
+  if constexpr (S::G > 1) {  // a block with one row group has nothing to share
+    if (w.coop) {
+      adaln_bwd_walk_kernel<TX, TY, 1, WPR, true, kBwdNT, NTL><<<w.blocks, S::BLK, 0, s>>>(a, o);
+      return check_launch("nf_adaln_bwd_full");
+    }
+  }
+  adaln_bwd_walk_kernel<TX, TY, 1, WPR, false, kBwdNT, NTL><<<w.blocks, S::BLK, 0, s>>>(a, o);
   return check_launch("nf_adaln_bwd_full");
+}
+template <typename TX, typename TY, int WPR>
+int launch_walk_t(const BwdArgs &a, const WalkOut &o, const WalkPlan &w, hipStream_t s) {
+  if constexpr (sizeof(TX) == 2) {
+    if (nt_loads_for(a.M * a.N * bwd_row_bytes<TX, TY>(a)))
+      return launch_walk_c<TX, TY, WPR, true>(a, o, w, s);
+  }
+  return launch_walk_c<TX, TY, WPR, false>(a, o, w, s);
 }
 
 // (wavefronts per row, chunks per lane) pairs make_plan gives on the vector
@@ -1262,12 +1314,11 @@ int bwd_v(const BwdArgs &a, const Plan &pl, bool vec, hipStream_t s) {
 template <typename TX, typename TY>
 int bwd_walk(const BwdArgs &a, const WalkOut &o, const Plan &pl, const WalkPlan &w,
              hipStream_t s) {
-  if (pl.bwd_k == 2) return launch_walk_t<TX, TY, 8, 2>(a, o, w, s);
   switch (pl.bwd_wpr) {
-    case 1: return launch_walk_t<TX, TY, 1, 1>(a, o, w, s);
-    case 2: return launch_walk_t<TX, TY, 2, 1>(a, o, w, s);
-    case 4: return launch_walk_t<TX, TY, 4, 1>(a, o, w, s);
-    default: return launch_walk_t<TX, TY, 8, 1>(a, o, w, s);
+    case 1: return launch_walk_t<TX, TY, 1>(a, o, w, s);
+    case 2: return launch_walk_t<TX, TY, 2>(a, o, w, s);
+    case 4: return launch_walk_t<TX, TY, 4>(a, o, w, s);
+    default: return launch_walk_t<TX, TY, 8>(a, o, w, s);
   }
 }
 

@@ -16,6 +16,7 @@ import numpy as np
 import pytest
 import torch
 
+from nuvla_forge_amd import _lib
 from nuvla_forge_amd.kernels import fused_adaln_residual_rmsnorm
 from oracle import numerics as on
 from tests.helpers import TOL, gen, note, np64, randn
@@ -146,6 +147,77 @@ def test_adaln_backward_over_many_samples(cuda, xd, yd, b, t, n):
     got = torch.autograd.grad(outs, [leaves[k] for k in ("x", "shift", "weight")], [dh, dout])
     for k, v in zip(("x", "shift", "weight"), got):
         assert torch.equal(v, grads[k]), f"d{k} alone differs"
+
+
+@pytest.mark.parametrize("xd,yd,b,t,n", [
+    (torch.float32, torch.bfloat16, 1030, 33, 72),    # one sample a block past 1024 blocks
+    (torch.bfloat16, torch.bfloat16, 1100, 17, 520),  # groups share long samples of many
+    (torch.bfloat16, torch.bfloat16, 2100, 34, 136),  # two samples a block, shared
+    (torch.float32, torch.float32, 1600, 9, 1032),    # two samples a block, one row group
+    (torch.float32, torch.bfloat16, 300, 3, 4104),    # two chunks a lane: the row kernel
+])
+def test_adaln_backward_over_many_long_samples(cuda, xd, yd, b, t, n):
+    note(f"adaln many long samples {xd}/{yd} b={b} t={t} n={n}")
+    inp = _inputs(b, t, n, xd, cuda, cond_dtype=yd, y_dtype=yd)
+    dh, dout = _upstream(b * t, n, xd, cuda)
+    h, out, grads = _run(inp, t, dh, dout)
+    a = {k: np64(v) for k, v in inp.items()}
+    gw = on.adaln_backward(**a, t=t, dh_up=np64(dh), dout=np64(dout), eps=1e-6)
+    for k in NAMES:
+        assert on.rel_err(np64(grads[k]), gw[k]) <= TOL[grads[k].dtype], k
+    _, _, again = _run(inp, t, dh, dout)
+    for k in NAMES:
+        assert torch.equal(again[k], grads[k]), f"d{k} differs between runs"
+
+
+@pytest.mark.parametrize("b,t,n", [
+    (850, 100, 1024),  # the walk with hinted loads, its groups sharing a sample
+    (900, 21, 4096),   # the same, one row group a block
+    (600, 700, 264),   # the row kernel and the reduction
+    (260, 1300, 256),  # the same
+])
+def test_adaln_backward_over_many_samples_beyond_the_cache(cuda, b, t, n):
+    """bf16 operands beyond the Infinity Cache: nf_adaln_bwd_full against
+    nf_adaln_bwd and nf_adaln_bwd_reduce, whose sums run in another order."""
+    note(f"adaln many samples beyond the cache b={b} t={t} n={n}")
+    g = torch.Generator(device=cuda).manual_seed(b)
+    rnd = lambda *s, std=1.0: torch.randn(*s, device=cuda, generator=g).mul_(std).bfloat16()  # noqa: E731
+    m = b * t
+    assert 8 * m * n > 320 << 20
+    x, y, dh, dout = rnd(m, n), rnd(m, n), rnd(m, n), rnd(m, n)
+    gate, scale, w = rnd(b, n, std=0.1), rnd(b, n, std=0.1), rnd(n, std=0.02) + 1
+    rstd = (x.float() + gate.float().repeat_interleave(t, 0) * y.float()).square().mean(-1).rsqrt()
+    L, p = _lib.lib(), lambda v: v.data_ptr()  # noqa: E731
+    nb = L.nf_adaln_bwd_workspace(m, n, t)
+    code = _lib.dtype_code(torch.bfloat16)
+
+    def run(full):
+        ws = torch.empty(nb, dtype=torch.uint8, device=cuda)
+        out = [torch.empty_like(x), torch.empty_like(y), torch.empty_like(gate),
+               torch.empty_like(w), torch.empty_like(scale), torch.empty_like(scale)]
+        ins = (p(dh), p(dout), p(x), n, p(y), n, p(gate), n, p(w), p(scale), n, p(rstd))
+        par = [p(v) for v in out[2:]]
+        if full:
+            _lib.check(L.nf_adaln_bwd_full(*ins, p(out[0]), p(out[1]), *par, p(ws), nb, m, n, t,
+                                           *[code] * 6, _lib.stream_of(x)), "nf_adaln_bwd_full")
+        else:
+            _lib.check(L.nf_adaln_bwd(*ins, p(out[0]), p(out[1]), p(ws), nb, m, n, t,
+                                      *[code] * 5, _lib.stream_of(x)), "nf_adaln_bwd")
+            _lib.check(L.nf_adaln_bwd_reduce(p(ws), nb, p(w), p(scale), n, *par, m, n, t,
+                                             *[code] * 4, _lib.stream_of(x)), "nf_adaln_bwd_reduce")
+        torch.cuda.synchronize()
+        return out
+
+    got, want = run(True), run(False)
+    # one bf16 rounding each (an ulp, 2^-7, apart at most) of fp32 values a few
+    # roundings of a row apart: 2^-24 of terms below 64, 16 of them
+    for a, e in zip(got[:2], want[:2]):
+        assert ((a.float() - e.float()).abs() <= 2.0 ** -7 * e.float().abs() + 2.0 ** -14).all()
+    # sums of up to 1300 rows, dweight's of all: 2^-24 of the sum of the terms'
+    # sizes a step at most, far below the bf16 rounding in the norm
+    for a, e in zip(got[2:], want[2:]):
+        d = (a.double() - e.double()).norm() / e.double().norm()
+        assert d <= 2.0 ** -8, float(d)
 
 
 @pytest.mark.parametrize("yd,b,t,n", [
