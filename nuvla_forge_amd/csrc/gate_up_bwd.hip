@@ -289,6 +289,25 @@ inline bool under_2gib(int64_t rows, int64_t ld) {
 
 using namespace nf;
 
+// The line between the one launch and what it stands beside for bf16 (dx as two
+// library GEMMs, nf_gemm_swiglu_wgrad on transposed copies, dx's two terms
+// rounded in between).  The M- and N-major operands take twice the LDS reads of
+// K-contiguous ones, which costs more than transposing once the products are
+// long in all three extents and power-bound.  Forward + backward, us, one launch
+// against the other form:
+//   M 4096 D 2048 H 5632 627 / 656;   M 2048 D 3072 H 8192 665 / 668;
+//   M 8192 D 1536 H 8192 1336 / 1357; M 65536 D 2048 H 1536 2649 / 2779;
+//   M 4096 D 5120 H 2736 756 / 836;   M 1024 D 4096 H 11008 668 / 682;
+//   M 4096 D 3072 H 5632 912 / 898;   M 4096 D 2048 H 11008 1284 / 1190;
+//   M 8192 D 2048 H 5632 1302 / 1208; M 4096 D 4096 H 11008 2270 / 1970;
+//   M 16384 D 4096 H 5632 4398 / 3880; M 8192 D 8192 H 8192 5996 / 5202.
+// (The transposed copies, M padded to 8, must stay under 2 GiB.)
+extern "C" int nf_gemm_swiglu_bwd_wins(int64_t M, int64_t D, int64_t H) {
+  const bool large = M >= 2048 && D >= 2048 && H >= 2560 &&
+                     (double)M * (double)D * (double)H >= 6.5e10;
+  return !(large && gate_up::under_2gib(M + 7, H > D ? H : D));
+}
+
 extern "C" size_t nf_gemm_swiglu_bwd_workspace(int64_t M, int64_t D, int64_t H, int want_dx,
                                                int want_dgate, int want_dup) {
   const int64_t big = (int64_t)1 << 31;

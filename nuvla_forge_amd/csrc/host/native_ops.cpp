@@ -253,17 +253,37 @@ struct GateUp : torch::autograd::Function<GateUp> {
     const bool need_g = ctx->needs_input_grad(1), need_u = ctx->needs_input_grad(2);
     const auto tw = need_g && need_u && tg != tu ? at::kFloat : need_g ? tg : tu;
     Tensor dx, dg, du;
-    if (ctx->needs_input_grad(0)) dx = at::empty({m, d}, x.options().dtype(tx));
+    bool one_x = ctx->needs_input_grad(0), one_w = need_g || need_u;  // left to the one launch
     if (need_g) dg = at::empty({h, d}, x.options().dtype(tw));
     if (need_u) du = at::empty({h, d}, x.options().dtype(tw));
-    const size_t nb = nf_gemm_swiglu_bwd_workspace(m, d, h, dx.defined(), dg.defined(),
-                                                   du.defined());
-    Tensor ws = bytes(nb, x);
-    check(nf_gemm_swiglu_bwd(da.data_ptr(), db.data_ptr(), h, x.data_ptr(), x.stride(0),
-                             wg.data_ptr(), wg.stride(0), wu.data_ptr(), wu.stride(0), ptr(dx),
-                             code_of(tx), ptr(dg), ptr(du), code_of(tw), m, d, h, NF_DTYPE_BF16,
-                             ws.data_ptr(), nb, st),
-          "nf_gemm_swiglu_bwd");
+    if (tx == at::kBFloat16 && tg == tx && tu == tx && !nf_gemm_swiglu_bwd_wins(m, d, h)) {
+      if (one_x) {
+        const at::NoGradGuard no_grad;
+        const c10::impl::ExcludeDispatchKeyGuard no_autocast(c10::autocast_dispatch_keyset);
+        dx = at::addmm(at::mm(da, wg), db, wu);
+        one_x = false;
+      }
+      if (need_g && need_u) {
+        const size_t nb = nf_gemm_swiglu_wgrad_workspace(m, d, h);
+        Tensor ws = bytes(nb, x);
+        check(nf_gemm_swiglu_wgrad(da.data_ptr(), db.data_ptr(), h, x.data_ptr(), x.stride(0),
+                                   dg.data_ptr(), du.data_ptr(), d, m, d, h, NF_DTYPE_BF16,
+                                   ws.data_ptr(), nb, st),
+              "nf_gemm_swiglu_wgrad");
+        one_w = false;
+      }
+    }
+    if (one_x) dx = at::empty({m, d}, x.options().dtype(tx));
+    if (one_x || one_w) {
+      void *const pg = one_w ? ptr(dg) : nullptr, *const pu = one_w ? ptr(du) : nullptr;
+      const size_t nb = nf_gemm_swiglu_bwd_workspace(m, d, h, one_x, pg != nullptr, pu != nullptr);
+      Tensor ws = bytes(nb, x);
+      check(nf_gemm_swiglu_bwd(da.data_ptr(), db.data_ptr(), h, x.data_ptr(), x.stride(0),
+                               wg.data_ptr(), wg.stride(0), wu.data_ptr(), wu.stride(0),
+                               one_x ? dx.data_ptr() : nullptr, code_of(tx), pg, pu, code_of(tw),
+                               m, d, h, NF_DTYPE_BF16, ws.data_ptr(), nb, st),
+            "nf_gemm_swiglu_bwd");
+    }
     return {dx, need_g ? dg.to(tg) : dg, need_u ? du.to(tu) : du};
   }
 };

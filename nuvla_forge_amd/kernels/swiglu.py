@@ -75,7 +75,9 @@ class _FusedGateUpSwiGLU(torch.autograd.Function):
     backward: ``nf_swiglu_bwd`` forms da, db from a, b and dact (sigmoid
     recomputed); ``nf_gemm_swiglu_bwd`` computes dx = da W_gate + db W_up,
     dW_gate = da^T x and dW_up = db^T x in one launch, each written once in
-    its input's type (sums over K splits added in a fixed order).
+    its input's type (sums over K splits added in a fixed order).  Where
+    ``nf_gemm_swiglu_bwd_wins`` says no (large all-bf16 products), dx is two
+    library GEMMs and both weight gradients come from ``nf_gemm_swiglu_wgrad``.
     """
 
     @staticmethod
@@ -129,19 +131,38 @@ class _FusedGateUpSwiGLU(torch.autograd.Function):
         dx = torch.empty((m, d), dtype=cx, device=x.device) if need_x else None
         dwg = torch.empty((h, d), dtype=cw, device=x.device) if need_g else None
         dwu = torch.empty((h, d), dtype=cw, device=x.device) if need_u else None
+        code = _lib.dtype_code(torch.bfloat16)
+        one_x, one_w = need_x, need_g or need_u  # left to the one launch
         with device_of(x):
-            nbytes = L.nf_gemm_swiglu_bwd_workspace(m, d, h, need_x, need_g, need_u)
-            ws = torch.empty(max(nbytes, 1), dtype=torch.uint8, device=x.device)
-            _lib.check(
-                L.nf_gemm_swiglu_bwd(da.data_ptr(), db.data_ptr(), h, x.data_ptr(),
-                                     x.stride(0), w_gate.data_ptr(), w_gate.stride(0),
-                                     w_up.data_ptr(), w_up.stride(0), _lib.ptr(dx),
-                                     _lib.dtype_code(cx), _lib.ptr(dwg), _lib.ptr(dwu),
-                                     _lib.dtype_code(cw), m, d, h,
-                                     _lib.dtype_code(torch.bfloat16), ws.data_ptr(), nbytes,
-                                     _lib.stream_of(x)),
-                "nf_gemm_swiglu_bwd",
-            )
+            st = _lib.stream_of(x)
+            if tx == tg == tu == torch.bfloat16 and not L.nf_gemm_swiglu_bwd_wins(m, d, h):
+                if one_x:
+                    with torch.no_grad(), torch.autocast(x.device.type, enabled=False):
+                        dx = torch.addmm(torch.mm(da, w_gate), db, w_up)
+                    one_x = False
+                if need_g and need_u:
+                    nbytes = L.nf_gemm_swiglu_wgrad_workspace(m, d, h)
+                    ws = torch.empty(max(nbytes, 1), dtype=torch.uint8, device=x.device)
+                    _lib.check(
+                        L.nf_gemm_swiglu_wgrad(da.data_ptr(), db.data_ptr(), h, x.data_ptr(),
+                                               x.stride(0), dwg.data_ptr(), dwu.data_ptr(), d,
+                                               m, d, h, code, ws.data_ptr(), nbytes, st),
+                        "nf_gemm_swiglu_wgrad",
+                    )
+                    one_w = False
+            if one_x or one_w:
+                pg, pu = (_lib.ptr(dwg), _lib.ptr(dwu)) if one_w else (None, None)
+                nbytes = L.nf_gemm_swiglu_bwd_workspace(m, d, h, one_x, bool(pg), bool(pu))
+                ws = torch.empty(max(nbytes, 1), dtype=torch.uint8, device=x.device)
+                _lib.check(
+                    L.nf_gemm_swiglu_bwd(da.data_ptr(), db.data_ptr(), h, x.data_ptr(),
+                                         x.stride(0), w_gate.data_ptr(), w_gate.stride(0),
+                                         w_up.data_ptr(), w_up.stride(0),
+                                         dx.data_ptr() if one_x else None, _lib.dtype_code(cx),
+                                         pg, pu, _lib.dtype_code(cw), m, d, h, code,
+                                         ws.data_ptr(), nbytes, st),
+                    "nf_gemm_swiglu_bwd",
+                )
         return (dx.to(tx) if need_x else None, dwg.to(tg) if need_g else None,
                 dwu.to(tu) if need_u else None)
 

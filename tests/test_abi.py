@@ -178,6 +178,17 @@ def test_gemm_swiglu_wgrad_workspace_and_validation():
     assert L.nf_gemm_swiglu_wgrad_workspace(1 << 62, d, h) == 0
 
 
+@pytest.mark.parametrize("m,d,h,wins", [
+    (9408, 384, 1536, 1), (4096, 2048, 5632, 1), (65536, 2048, 1536, 1), (4096, 5120, 2736, 1),
+    (8192, 2048, 5632, 0), (4096, 4096, 11008, 0), (2048, 8192, 8192, 0),
+    (2047, 8192, 8192, 1),                  # below each of the line's sizes
+    (1 << 17, 2048, 8191, 0),               # the operands still under 2 GiB ...
+    ((1 << 17) - 3, 2048, 8192, 1),         # ... and the padded copies no longer
+    (0, 4096, 4096, 1)])
+def test_gemm_swiglu_bwd_wins_where_it_was_measured_to(m, d, h, wins):
+    assert _lib.lib().nf_gemm_swiglu_bwd_wins(m, d, h) == wins
+
+
 def test_adaln_argument_validation():
     L = _lib.lib()
     args = [FAKE, 1024, FAKE, 1024, FAKE, 1024, FAKE, FAKE, 1024, FAKE, 1024, FAKE, FAKE, FAKE]

@@ -160,6 +160,30 @@ def test_gate_up_gradients_in_any_input_types(cuda, xd, gd, ud, need):
     _same(got, [v.to(t) for v, t in zip(want, types)])
 
 
+@pytest.mark.parametrize("need", [(True, True, True), (True, False, False), (False, True, True),
+                                  (True, False, True)])
+def test_gate_up_large_products(cuda, need):
+    """Above the line of nf_gemm_swiglu_bwd_wins: both hosts alike, and each
+    gradient against fp32 products of the same bf16 inputs."""
+    m, d, h = 2056, 4096, 8200
+    note(f"gate/up large m={m} d={d} h={h} need={need}")
+    assert not _lib.lib().nf_gemm_swiglu_bwd_wins(m, d, h)
+    g = torch.Generator(device=cuda).manual_seed(12)
+    rnd = lambda *s, std=1.0: torch.randn(*s, device=cuda, generator=g).mul_(std).bfloat16()  # noqa: E731
+    inputs = [rnd(m, d), rnd(h, d, std=d ** -0.5), rnd(h, d, std=d ** -0.5)]
+    up = [rnd(m, h)]
+    got = _grads(fused_gate_up_swiglu, inputs, need, up)
+    _same(got, _grads(swiglu._FusedGateUpSwiGLU.apply, inputs, need, up))
+    f = lambda x, wg, wu: torch.nn.functional.silu(x @ wg.T) * (x @ wu.T)  # noqa: E731
+    want = _grads(f, [v.float() for v in inputs], need, [up[0].float()])
+    # a, b, da, db, act, dx's partial sum and the gradients are rounded to bf16
+    # (2^-9 of each at most, about half that in the norm), at most five of
+    # them in a row and independent: sqrt(5) 2^-9
+    for a, e in zip(got, want):
+        assert a.dtype == BF16
+        assert (a.float() - e).norm() <= 5 ** 0.5 * 2.0 ** -9 * e.norm()
+
+
 @pytest.mark.parametrize("m,d,h", [(300, 136, 264), (5, 64, 1000), (300, 36, 100)])
 @pytest.mark.parametrize("dtype", [BF16, F32])
 def test_gate_up_without_a_backward(cuda, m, d, h, dtype):
