@@ -224,7 +224,9 @@ __global__ __launch_bounds__(kSumThreads) void gate_up_reduce_kernel(Sums p) {
 // K splits of the launch.  nx dx tiles of kx stages and nw dW tiles of kw
 // stages run on 256 CUs, one block each, the longer blocks first; a block
 // also costs ~4 stages of prologue and epilogue, and a split product the
-// write and read of its fp32 slices (stages of ~1.8 us against ~5 TB/s).
+// write and read of its fp32 slices (stages of ~1.8 us against ~5 TB/s).  A few
+// tokens against a wide H leave one or two dx tiles of all K: M 48 D 256 H 11008,
+// forward + backward, 103 us with at most 8 dx slices, 55 with up to 32.
 struct Split {
   int sx, sw;
 };
@@ -236,7 +238,7 @@ inline Split pick_split(int64_t M, int64_t D, int64_t H, bool want_x, int want_w
   const double over = 4.0, per_byte = 1.0 / (5e12 * 1.8e-6);
   Split best{1, 1};
   double best_t = -1.0;
-  for (int sx = 1; sx <= 8 && (sx == 1 || (want_x && kx / sx >= 4)); ++sx)
+  for (int sx = 1; sx <= 32 && (sx == 1 || (want_x && kx / sx >= 4)); sx += sx < 8 ? 1 : sx / 4)
     for (int sw = 1; sw <= 32 && (sw == 1 || (want_w && kw / sw >= 4)); ++sw) {
       const double lx = (double)((kx + sx - 1) / sx) + over, lw = (double)((kw + sw - 1) / sw) + over;
       double t = lx >= lw ? gemm::two_job_makespan(nx * sx, lx, nw * sw, lw)

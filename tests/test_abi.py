@@ -178,6 +178,33 @@ def test_gemm_swiglu_wgrad_workspace_and_validation():
     assert L.nf_gemm_swiglu_wgrad_workspace(1 << 62, d, h) == 0
 
 
+def test_gemm_swiglu_bwd_workspace_and_validation():
+    L = _lib.lib()
+    m, d, h = 700, 200, 1000
+    size = L.nf_gemm_swiglu_bwd_workspace
+    want = size(m, d, h, 1, 1, 1)
+    assert want > 0 and size(m, d, h, 0, 0, 0) == 0
+    assert size(0, d, h, 1, 1, 1) == 0 and size(1 << 62, d, h, 1, 1, 1) == 0
+
+    def call(**kw):
+        a = dict(da=FAKE, db=FAKE, ld_ab=h, x=FAKE, ldx=d, wg=FAKE, ld_gate=d, wu=FAKE, ld_up=d,
+                 dx=FAKE, dt_dx=0, dwg=FAKE, dwu=FAKE, dt_dw=1, m=m, d=d, h=h, dtype=1, ws=FAKE,
+                 nbytes=want) | kw
+        return L.nf_gemm_swiglu_bwd(*a.values(), None)
+
+    assert call(d=0) == NF_ERR_ARG and "bad shape" in _err()
+    assert call(dtype=0) == NF_ERR_DTYPE and "bf16 only" in _err()
+    assert call(dt_dx=7) == NF_ERR_DTYPE and call(dt_dw=-1) == NF_ERR_DTYPE
+    for null in ("da", "db", "x", "wg", "wu"):
+        assert call(**{null: None}) == NF_ERR_ARG and "null" in _err()
+    for short in (dict(ld_ab=h - 1), dict(ldx=d - 1), dict(ld_gate=d - 1), dict(ld_up=d - 1)):
+        assert call(**short) == NF_ERR_ARG and "leading dimension" in _err()
+    assert call(ld_ab=1 << 22) == NF_ERR_ARG and "2 GiB" in _err()
+    for bad in (dict(ws=None), dict(nbytes=want - 1), dict(ws=FAKE + 4)):
+        assert call(**bad) == NF_ERR_WORKSPACE and str(want) in _err()
+    assert call(dx=None, dwg=None, dwu=None, ws=None, nbytes=0) == NF_OK  # nothing wanted
+
+
 @pytest.mark.parametrize("m,d,h,wins", [
     (9408, 384, 1536, 1), (4096, 2048, 5632, 1), (65536, 2048, 1536, 1), (4096, 5120, 2736, 1),
     (8192, 2048, 5632, 0), (4096, 4096, 11008, 0), (2048, 8192, 8192, 0),

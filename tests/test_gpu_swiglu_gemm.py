@@ -225,6 +225,94 @@ def test_gate_up_wgrad_entry_without_tokens_zeroes(cuda):
     assert bool((dwg[:, 32:] == 7.0).all())
 
 
+def _bwd(da, db, x, wg, wu, dt, want=(True, True, True)):
+    """nf_gemm_swiglu_bwd on row-strided views, its gradients (or None) in `dt`
+    in buffers of NaN, and its workspace's size."""
+    m, h = da.shape
+    d = wg.shape[1]
+    out = [torch.full(s, float("nan"), dtype=dt, device=wg.device) if k else None
+           for s, k in zip(((m, d), (h, d), (h, d)), want)]
+    L, code, dc = _lib.lib(), _lib.dtype_code(torch.bfloat16), _lib.dtype_code(dt)
+    nb = L.nf_gemm_swiglu_bwd_workspace(m, d, h, *want)
+    ws = torch.full((max(nb, 1),), 255, dtype=torch.uint8, device=wg.device)
+    _lib.check(L.nf_gemm_swiglu_bwd(da.data_ptr(), db.data_ptr(), da.stride(0), x.data_ptr(),
+                                    x.stride(0), wg.data_ptr(), wg.stride(0), wu.data_ptr(),
+                                    wu.stride(0), _lib.ptr(out[0]), dc, _lib.ptr(out[1]),
+                                    _lib.ptr(out[2]), dc, m, d, h, code, ws.data_ptr(), nb,
+                                    _lib.stream_of(wg)), "nf_gemm_swiglu_bwd")
+    torch.cuda.synchronize()
+    return out, nb
+
+
+def _bwd_inputs(m, d, h, pad, dev, seed):
+    """da, db, x, w_gate, w_up as views whose rows end in `pad` NaN (w_up: twice)."""
+    g = gen(seed)
+
+    def view(rows, cols, extra, std=1.0):
+        t = torch.full((rows, cols + extra), float("nan"), dtype=torch.bfloat16)
+        t[:, :cols] = randn((rows, cols), g, torch.bfloat16, "cpu", std=std)
+        return t.to(dev)[:, :cols]
+
+    return [view(m, h, pad), view(m, h, pad), view(m, d, pad), view(h, d, pad, d ** -0.5),
+            view(h, d, 2 * pad, d ** -0.5)]
+
+
+# tile edges (256) and remainders, slices of dx's K across the seam between the
+# gate and the up units (an odd number of 64-deep stages each), more than 8 dx
+# slices, ragged last slices of both products, rows that are not whole vectors
+# (element-wise copies and stores), one token, one unit
+@pytest.mark.parametrize("m,d,h,pad,sx,sw", [
+    (256, 256, 256, 0, True, False), (257, 264, 328, 8, True, False),
+    (40, 72, 4104, 0, True, False), (3000, 136, 264, 8, True, True),
+    (700, 200, 1000, 16, True, True), (300, 37, 101, 3, False, False),
+    (1100, 36, 700, 0, True, True), (1, 8, 8, 0, False, False), (513, 520, 1, 7, False, True)])
+def test_gate_up_bwd_entry_matches_fp64(cuda, m, d, h, pad, sx, sw):
+    """dx = da W_gate + db W_up, dW_gate = da^T x, dW_up = db^T x in fp32 from the
+    same bf16 operands in fp64, element by element; a second call gives the
+    same bits, and bf16 results are the fp32 ones rounded once."""
+    note(f"gate/up bwd entry m={m} d={d} h={h} pad={pad}")
+    ops = _bwd_inputs(m, d, h, pad, cuda, m + d)
+    da, db, x, wg, wu = (t.double() for t in ops)
+    L = _lib.lib()
+    assert (L.nf_gemm_swiglu_bwd_workspace(m, d, h, 1, 0, 0) > 0) == sx
+    assert (L.nf_gemm_swiglu_bwd_workspace(m, d, h, 0, 1, 0) > 0) == sw
+    got, _ = _bwd(*ops, torch.float32)
+    want = [da @ wg + db @ wu, da.T @ x, db.T @ x]
+    size = [da.abs() @ wg.abs() + db.abs() @ wu.abs(), da.abs().T @ x.abs(), db.abs().T @ x.abs()]
+    # an accumulator takes K / 16 MFMAs of a few roundings each (4 are taken),
+    # each 2^-24 of at most the sum of the products' sizes, then the slices' sum
+    for v, w, z, k in zip(got, want, size, (2 * (h + 64), m + 64, m + 64)):
+        assert ((v.double() - w).abs() <= (k / 4 + 33) * 2.0 ** -24 * z).all()
+    again, _ = _bwd(*ops, torch.float32)
+    half, _ = _bwd(*ops, torch.bfloat16)
+    for v, a, b in zip(got, again, half):
+        assert torch.equal(v, a) and torch.equal(v.bfloat16(), b)
+
+
+@pytest.mark.parametrize("want", [(True, False, False), (False, True, False), (False, False, True),
+                                  (True, True, False), (False, True, True), (False, False, False)])
+def test_gate_up_bwd_entry_writes_what_is_wanted(cuda, want):
+    """Any subset of the gradients: the values of a call for all three (their K
+    split may differ: an fp32 sum in another order)."""
+    m, d, h = 700, 200, 1000
+    note(f"gate/up bwd entry subset {want}")
+    ops = _bwd_inputs(m, d, h, 0, cuda, 5)
+    every, _ = _bwd(*ops, torch.float32)
+    got, _ = _bwd(*ops, torch.float32, want)
+    for v, e, k in zip(got, every, want):
+        assert (v is not None) == k
+        if k:
+            assert (v - e).norm() <= 1e-6 * e.norm()
+
+
+@pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16, torch.float16])
+def test_gate_up_bwd_entry_without_tokens_zeroes(cuda, dt):
+    note(f"gate/up bwd entry m=0 {dt}")
+    ops = _bwd_inputs(0, 40, 24, 0, cuda, 6)
+    (dx, dwg, dwu), _ = _bwd(*ops, dt)
+    assert dx.numel() == 0 and (dwg == 0).all() and (dwu == 0).all()
+
+
 def test_gate_up_fwd_bwd_replays_in_a_graph(cuda):
     """The encoder-MLP gate/up step (GEMM with the SwiGLU epilogue, SwiGLU
     backward, split-K weight gradients with their transposes and reduce, dx)
