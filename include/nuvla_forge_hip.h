@@ -239,7 +239,9 @@ int nf_adaln_bwd_noalloc(const void *dh_up, const void *dout, const void *x,
  * *bad_targets (device int32, may be NULL) and treated as ignored.
  * hidden [M, D] and weight [V, D] are contiguous and share `dtype`
  * (NF_DTYPE_BF16 uses bf16 MFMA with fp32 accumulation, NF_DTYPE_F32 six
- * bf16 products over three-part operands, more precise than fp32 MFMA).  targets is int64 [M].
+ * bf16 products over three-part operands, whose norm-wise error is below fp32
+ * MFMA's; of values under 2^-110 they keep 2^-134, not 2^-149).  targets is
+ * int64 [M].
  *
  * Only valid rows do work: the forward compacts them on the device (the
  * count never reaches the host) and forms each row's logits once, so the

@@ -6,7 +6,7 @@
 //    K-contiguous, four v_mfma_f32_16x16x32_bf16 per 32x32 tile brought to
 //    the same accumulator layout (mainloop_dtl16).
 //  * f32 inputs are split into three bf16 parts and multiplied as six bf16
-//    products (SplitCfg, mainloop_split), more precise than the fp32 MFMAs at
+//    products (SplitCfg, mainloop_split), with a smaller error than the fp32 MFMAs at
 //    over twice their rate.
 //  * Accumulator (32x32, 16 fp32 per lane): register r of lane l holds
 //    row 8 * (r / 4) + 4 * (l / 32) + (r % 4), column l % 32.
@@ -732,9 +732,10 @@ __device__ __forceinline__ void mainloop_dtl_ops(const OpA &opa, const OpB &opb,
 // ---- fp32 operands as three bf16 parts (SplitCfg) ------------------------------
 // A finite fp32 value is the sum of three bf16 values: b1 its leading 8
 // significant bits (truncated, so nothing overflows), b2 the next 8 of the
-// remainder (rounded) and b3 what is left (exact).  The product of two values
+// remainder (rounded) and b3 what is left (exact; values below 2^-110 keep what
+// bf16's last subnormal bit leaves, to 2^-134).  The product of two values
 // is taken as b1 c1 + (b1 c2 + b2 c1 + b1 c3 + b3 c1 + b2 c2); what is left
-// out is below 2^-24 of it, with either sign.  The six products run on
+// out is below 2^-22 of it, with either sign.  The six products run on
 // v_mfma_f32_16x16x32_bf16, b1 c1 into one accumulator and the five small ones
 // into another (their roundings are then below the first's by 2^-7), added at
 // the end.  Each MFMA adds 32 products to the accumulator with fewer fp32
@@ -779,19 +780,24 @@ struct SplitCfg {
 // serves together into 16 different 16-byte columns of the banks.
 __device__ __forceinline__ int split_slot(int row, int kv) { return kv ^ ((row >> 2) & 2); }
 
+// v_cmp_class bits: NaNs (0, 1) and subnormals (4, 7)
+constexpr int kOddClass = 0x1 | 0x2 | 0x10 | 0x80;
+
 // 8 fp32 (two 16-byte vectors) -> the three parts, 8 bf16 each
 __device__ __forceinline__ void split8(const u32x4 (&x)[2], u32x4 (&part)[3]) {
   typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 #pragma unroll
   for (int p = 0; p < 4; ++p) {  // pairs
     const uint32_t u0 = x[p >> 1][2 * (p & 1)], u1 = x[p >> 1][2 * (p & 1) + 1];
+    // a subnormal's or a NaN's last bit is set: no value but zero has a zero first
+    // part, and a NaN with payload in its low bits only stays one.  What is left
+    // of an infinity is a NaN: its products are infinite without it
+    // (mainloop_split leaves the others out there)
     const float f0 = __uint_as_float(u0), f1 = __uint_as_float(u1);
-    // quieted first: a NaN with payload in its low bits only would be cut to an infinity
-    const uint32_t h0 = __float_as_uint(__builtin_canonicalizef(f0)) & 0xffff0000u;
-    const uint32_t h1 = __float_as_uint(__builtin_canonicalizef(f1)) & 0xffff0000u;
-    // an infinity is its own first part, with nothing left
-    const float r0 = (u0 & 0x7fffffffu) == 0x7f800000u ? 0.f : f0 - __uint_as_float(h0);
-    const float r1 = (u1 & 0x7fffffffu) == 0x7f800000u ? 0.f : f1 - __uint_as_float(h1);
+    const uint32_t h0 = (u0 & 0xffff0000u) | (__builtin_amdgcn_classf(f0, kOddClass) ? 0x10000u : 0u);
+    const uint32_t h1 = (u1 & 0xffff0000u) | (__builtin_amdgcn_classf(f1, kOddClass) ? 0x10000u : 0u);
+    const float r0 = f0 - __uint_as_float(h0);
+    const float r1 = f1 - __uint_as_float(h1);
     part[0][p] = (h0 >> 16) | h1;
     const bf16x2 m = {static_cast<__bf16>(r0), static_cast<__bf16>(r1)};
     const uint32_t mb = __builtin_bit_cast(uint32_t, m);

@@ -42,8 +42,9 @@ on chunk_size beyond fp rounding.
 Element types: under bf16 autocast for the device the products run in bf16
 (MFMA, fp32 accumulation) whatever the input types, as the reference's
 autocast-ed ``F.linear`` and ``@`` do; otherwise bf16 inputs run bf16 MFMA,
-fp32 inputs six bf16 products over three-part operands (more precise than fp32
-MFMA), and mixed or fp16 inputs are widened to fp32.
+fp32 inputs six bf16 products over three-part operands (a norm-wise error below
+fp32 MFMA's; of values under 2^-110 they keep 2^-134), and mixed or fp16 inputs
+are widened to fp32.
 """
 
 from __future__ import annotations

@@ -71,6 +71,40 @@ def test_split_gemm_keeps_infinities_and_nan(cuda):
     assert (got[3] == 16.0).all()
 
 
+def test_split_gemm_of_infinities_and_the_smallest_values(cuda):
+    """An infinity times any value but zero is an infinity, also where the value
+    is below the last subnormal of the parts' type (2^-133)."""
+    note("split gemm: inf times subnormals")
+    inf = float("inf")
+    a = torch.zeros(2, 32, device=cuda)
+    a[0, 9], a[1, 9] = inf, -inf
+    vals = torch.tensor([2.0 ** -126, 3 * 2.0 ** -134, 2.0 ** -134, 2.0 ** -140, -(2.0 ** -149),
+                         2.0 ** -149, 0.0, -1.0], device=cuda)
+    b = torch.zeros(len(vals), 32, device=cuda)
+    b[:, 9] = vals
+    got = _gemm(a, b, 32)
+    want = torch.tensor([inf, -inf], device=cuda)[:, None] * vals
+    assert torch.equal(got.isnan(), want.isnan()) and want.isnan().sum() == 2
+    assert torch.equal(got.nan_to_num(), want.nan_to_num())
+
+
+# Each operand in turn with parts that leave the most out: beside an exact
+# leading part, a second and a third part of the largest size and one sign
+@pytest.mark.parametrize("v", [1 + 2.0 ** -7 - 2.0 ** -15 + 2.0 ** -16 - 2.0 ** -23,
+                               1 + 2.0 ** -8 + 2.0 ** -16 + 2.0 ** -17, 2 - 2.0 ** -23,
+                               1 + 2.0 ** -7 - 2.0 ** -16 - 2.0 ** -23])
+@pytest.mark.parametrize("scale", [1.0, 2.0 ** -90, 2.0 ** -112])
+def test_split_gemm_of_operands_that_leave_the_most_out(cuda, v, scale):
+    """Eight equal products: 2^-22 of them left out, 4 roundings of 2^-24, and
+    2^-134 of each operand lost below 2^-110."""
+    note(f"split gemm: large remainders {v!r} x {scale}")
+    a, b = torch.zeros(5, 32, device=cuda), torch.zeros(7, 32, device=cuda)
+    a[:, 4:12], b[:, 4:12] = v * scale, v
+    got, A, B = np64(_gemm(a, b, 32)), np64(a), np64(b)
+    bound = 8 * 2.0 ** -24 * (A @ B.T) + 8 * 2.0 ** -134 * v
+    assert (np.abs(got - A @ B.T) <= bound).all()
+
+
 # signalling NaNs, positive and negative, whose payload lies in the 16 bits
 # below the first part
 @pytest.mark.parametrize("bits", [0x7f800001, 0x7f80ffff, 0xff800001 - (1 << 32)])
