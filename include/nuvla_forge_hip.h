@@ -256,7 +256,8 @@ int nf_adaln_bwd_noalloc(const void *dh_up, const void *dout, const void *x,
  * inv; results do not depend on chunk_rows beyond fp rounding.  bf16 keeps
  * a chunk's logits and the fp32 dweight accumulator together within the
  * bytes the reference's row chunks hold for them (an fp32 [chunk_rows, V]
- * tile and an fp32 [V, D] accumulator, up to 256-row rounding): one chunk
+ * tile and an fp32 [V, D] accumulator, up to 256-row rounding and rows of
+ * whole 128-byte lines): one chunk
  * over every row with no accumulator where that fits (logits held in both
  * layouts the products read for D >= 2048 when those fit, otherwise once,
  * row-major, the dweight product reading them transposed), else chunks of

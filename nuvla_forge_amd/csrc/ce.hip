@@ -43,6 +43,7 @@
 // plus the fp32 dW accumulator when there is more than one chunk; E and the
 // accumulator stay within the bytes the reference's chunk loop holds for
 // them (see make_plan), so E covers every row at once only where that fits.
+#include <initializer_list>
 #include <type_traits>
 
 #include "gemm_store.h"
@@ -808,13 +809,19 @@ struct Plan {
   size_t b_part, b_total;
 };
 
-// Row stride, in elements of `es` bytes, of a matrix whose rows are read in
+// Row stride, in elements of `es` bytes, of matrices whose rows are read in
 // 128-byte K slices: whole 128-byte lines once that pads a row by less than
 // 1.6%, so a slice is one line and not parts of two.  V 50001 and M 12289 at
 // D 384, forward + backward: 2.39 ms with padded rows, 2.61 with rows of whole
-// 16-byte vectors.
-inline int64_t line_stride(int64_t n, size_t es) {
-  return n < 4096 ? round_up(n, 8) : round_up(n, 128 / (int64_t)es);
+// 16-byte vectors.  column_bytes: what a column takes in each of the matrices; a
+// matrix that only the padding would take past the 2 GiB of buffer addressing
+// (element-wise copies from there on) keeps rows of whole vectors.
+inline int64_t line_stride(int64_t n, size_t es, std::initializer_list<int64_t> column_bytes) {
+  const int64_t plain = round_up(n, 8);
+  const int64_t lines = n < 4096 ? plain : round_up(n, 128 / (int64_t)es);
+  for (int64_t b : column_bytes)
+    if (sb_ok(plain * b) && !sb_ok(lines * b)) return plain;
+  return lines;
 }
 
 template <typename TI>
@@ -852,9 +859,10 @@ inline Plan plan_shape(int64_t M, int64_t D, int64_t V, int64_t chunk_rows) {
     P.crows = cr > mcap ? mcap : cr;
   }
   P.nch = (M + P.crows - 1) / P.crows;
-  P.ldp = line_stride(V, es);
+  const int64_t eb = (int64_t)es;
+  P.ldp = line_stride(V, es, {P.crows * eb, D * eb, P.single && P.nch > 1 ? D * 4 : 0});
   P.ldwt = P.ldp;
-  P.ldht = line_stride(M, es);
+  P.ldht = line_stride(M, es, {D * eb});
   P.wtm = C::WTM;
   P.vtiles = (int)((V + C::BM - 1) / C::BM);
   P.ntiles = P.vtiles * C::WM;

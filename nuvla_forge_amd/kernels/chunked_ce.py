@@ -30,7 +30,8 @@ loop in ATen (chunked_ce.py:133-167 with ``_ce_chunk_torch``, :101-117).
 ``chunk_size`` bounds memory by what the reference's row-chunk loop holds at
 the same setting: in bf16 a chunk's probabilities and the fp32 dW
 accumulator together stay within the bytes of its fp32 [chunk_size, V]
-logits tile plus its fp32 [V, D] dW accumulator (up to 256-row rounding).
+logits tile plus its fp32 [V, D] dW accumulator (up to 256-row rounding and,
+from V 4096 on, rows of whole 128-byte lines: 1.6 % at most).
 Where the probabilities of every row fit that, one chunk takes them all with
 no accumulator (held once, or for D >= 2048 in both layouts the gradient
 products read when those fit); otherwise chunks of 2 * chunk_size valid

@@ -265,10 +265,19 @@ def _ceil(a: int, b: int) -> int:
     return -(-a // b)
 
 
+def _ce_stride(n, es, column_bytes):
+    """A row stride of the CE's matrices: whole 16-byte vectors of 8 elements,
+    from 4096 on whole 128-byte lines, unless only that padding takes one of the
+    matrices (bytes a column) past 2 GiB."""
+    plain, lim = _ceil(n, 8) * 8, (1 << 31) - 64
+    lines = plain if n < 4096 else _ceil(n, 128 // es) * (128 // es)
+    return plain if any(plain * b < lim <= lines * b for b in column_bytes) else lines
+
+
 def _ce_state_closed_form(m, d, v, chunk_rows, es=2):
     """The state nf_ce_fwd leaves for nf_ce_bwd, term by term (each buffer
-    256-byte aligned): scalars, pos [M], the fp32 row factors [M], W^T
-    [D, V8], the scaled Hc^T [D, M8], one chunk's E, fp32 dH rows [M, D], and
+    256-byte aligned; V8 and M8 padded as in _ce_stride): scalars, pos [M], the
+    fp32 row factors [M], W^T [D, V8], the scaled Hc^T [D, M8], one chunk's E, fp32 dH rows [M, D], and
     the fp32 dW accumulator when more than one chunk.  bf16 (es 2) has a
     budget of 2 * (min(chunk_rows, M) + D) rows of E (the bytes of the
     reference's fp32 [chunk_rows, V] tile and fp32 [V, D] accumulator) and
@@ -288,8 +297,9 @@ def _ce_state_closed_form(m, d, v, chunk_rows, es=2):
     else:
         single = False
         c = min(a(want), mcap)
-    v8, m8 = _ceil(v, 8) * 8, _ceil(m, 8) * 8
     nch = _ceil(m, c)
+    v8 = _ce_stride(v, es, [es * c, es * d, 4 * d if single and nch > 1 else 0])
+    m8 = _ce_stride(m, es, [es * d])
     e_bytes = a(es * c * v8) + (0 if single else a(es * v * c))
     acc = (a(4 * d * v8) if single else a(4 * v * d)) if nch > 1 else 0
     return (a(64) + a(4 * m) + a(4 * m) + a(es * d * v8) + a(es * d * m8) + e_bytes
@@ -304,17 +314,20 @@ def test_ce_state_and_workspace_sizes():
     L = _lib.lib()
     shapes = [(4096, 2048, 32000, 1024), (4096, 2048, 32000, 4096), (4096, 4096, 32000, 4096),
               (4096, 4096, 32000, 1024), (16384, 2048, 32000, 1024), (16384, 384, 32000, 1024),
-              (512, 384, 32000, 1024), (300, 72, 1030, 100), (17, 36, 333, 7)]
+              (512, 384, 32000, 1024), (300, 72, 1030, 100), (17, 36, 333, 7),
+              # rows padded to whole 128-byte lines: V, M, both, neither
+              (1000, 384, 5000, 64), (4097, 200, 1000, 512), (12289, 384, 50001, 1024),
+              (4095, 40, 4095, 4096)]
     for m, d, v, cr in shapes:
         assert L.nf_ce_state_bytes(m, d, v, cr, 1) == _ce_state_closed_form(m, d, v, cr), (m, cr)
         assert L.nf_ce_state_bytes(m, d, v, cr, 0) == _ce_state_closed_form(m, d, v, cr, es=4)
     # bf16: E and the dW accumulator together stay within what the
     # reference's chunk loop holds for the same roles at the same chunk_size
     # (an fp32 [chunk_size, V] tile, an fp32 [V, D] accumulator), up to the
-    # rounding of a chunk to 256 rows
+    # rounding of a chunk to 256 rows and of a row to whole lines
     for m, d, v, cr in shapes:
         a = lambda x: _ceil(x, 256) * 256  # noqa: E731
-        v8, m8 = _ceil(v, 8) * 8, _ceil(m, 8) * 8
+        v8, m8 = _ce_stride(v, 2, []), _ce_stride(m, 2, [])
         rest = a(64) + 2 * a(4 * m) + a(2 * d * v8) + a(2 * d * m8) + a(4 * m * d)
         e_acc = L.nf_ce_state_bytes(m, d, v, cr, 1) - rest
         assert e_acc <= 4 * v8 * (min(cr, m) + d) + 4 * 256 * v8 + 512, (m, d, cr)
@@ -335,6 +348,26 @@ def test_ce_state_and_workspace_sizes():
     bws = L.nf_ce_bwd_workspace(4096, 2048, 32000, 1024, 1)
     assert fws > 4096 * 2048 * 2 and bws > 0  # the forward holds the gathered rows
     assert L.nf_ce_workspace(4096, 2048, 32000, 1024, 1) == sb + max(fws, bws)
+
+
+@pytest.mark.parametrize("m,d,v,chunk,es", [
+    (8192, 512, 131041, 8192, 2),     # E
+    (300, 8192, 131041, 300, 2),      # W^T
+    (20000, 8190, 65537, 1, 2),       # the dW accumulator [D, V8], in chunks
+    (131041, 8192, 1000, 1024, 2),    # Hc^T
+    (4096, 512, 131041, 4096, 4)])    # fp32 E
+def test_ce_padding_takes_no_matrix_past_2gib(m, d, v, chunk, es):
+    """Rows are not padded to lines where that alone would take a matrix out of
+    the kernels' 32-bit buffer addressing."""
+    L = _lib.lib()
+    got = L.nf_ce_state_bytes(m, d, v, chunk, 1 if es == 2 else 0)
+    assert got == _ce_state_closed_form(m, d, v, chunk, es)
+    lines = lambda n: _ceil(n, 128 // es) * (128 // es)  # noqa: E731
+    n = max(m, v)
+    assert lines(n) > _ceil(n, 8) * 8
+    # one column more of padding would be worth this much, at the least
+    assert got < _ce_state_closed_form(lines(m) if m == n else m, d, lines(v) if v == n else v,
+                                       chunk, es)
 
 
 def test_ce_argument_validation():

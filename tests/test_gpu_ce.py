@@ -369,6 +369,45 @@ def test_ce_one_call_entry_point(cuda, dtype, chunk_rows):
     assert torch.equal(loss, loss2) and torch.equal(dh, dh2) and torch.equal(dw, dw2)
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("m,d,v,chunk_rows", [
+    (4101, 40, 4999, 4101),   # rows of E, W^T and Hc^T padded to lines, one chunk
+    (4999, 72, 4101, 512),    # several chunks, the accumulator padded too
+    (4097, 384, 4097, 1024),  # 192-wide tiles, one element past the line's start
+    (300, 2048, 5003, 300),   # both layouts (bf16)
+    (4095, 33, 4095, 4096),   # the last sizes without padding, unaligned rows
+])
+def test_ce_rows_padded_to_lines(cuda, dtype, m, d, v, chunk_rows):
+    """Odd V and M around 4096, where rows start to be padded to whole 128-byte
+    lines, against float64; state and scratch start as NaN, so padding that a
+    product reads must have been written."""
+    note(f"ce padded rows dtype={dtype} m={m} d={d} v={v} chunk_rows={chunk_rows}")
+    hid, w, tgt = _ce_inputs(m, d, v, dtype, cuda, seed=21, w_std=2.0 * d ** -0.5,
+                             ignore=slice(None, None, 5))
+    L, code, f32 = _lib.lib(), _lib.dtype_code(dtype), _lib.dtype_code(torch.float32)
+    shape, s = (m, d, v, chunk_rows, code), _lib.stream_of(hid)
+
+    def poisoned(n):
+        return torch.full((n,), 255, dtype=torch.uint8, device=cuda), n
+
+    state, fws, bws = (poisoned(f(*shape)) for f in (L.nf_ce_state_bytes, L.nf_ce_fwd_workspace,
+                                                     L.nf_ce_bwd_workspace))
+    loss = torch.empty((), device=cuda)
+    dh, dw = torch.empty(m, d, device=cuda), torch.empty(v, d, device=cuda)
+    _lib.check(L.nf_ce_fwd(hid.data_ptr(), w.data_ptr(), tgt.data_ptr(), m, d, v, -100, chunk_rows,
+                           code, loss.data_ptr(), None, state[0].data_ptr(), state[1],
+                           fws[0].data_ptr(), fws[1], s), "nf_ce_fwd")
+    _lib.check(L.nf_ce_bwd(*shape, state[0].data_ptr(), state[1], None, dh.data_ptr(), f32,
+                           dw.data_ptr(), f32, bws[0].data_ptr(), bws[1], s), "nf_ce_bwd")
+    leaves = [t.double().requires_grad_(True) for t in (hid, w)]
+    want = torch.nn.functional.cross_entropy(leaves[0] @ leaves[1].T, tgt)
+    dhw, dww = torch.autograd.grad(want, leaves)
+    want = float(want.detach())
+    assert abs(float(loss) - want) <= TOL[dtype] * want
+    for got, exact in ((dh, dhw), (dw, dww)):
+        assert (got.double() - exact).norm() <= TOL[dtype] * exact.norm()
+
+
 def test_ce_grad_output_scaling(cuda):
     note("ce grad scaling")
     hid, w, tgt = _ce_inputs(128, 64, 500, torch.float32, cuda, seed=5)
