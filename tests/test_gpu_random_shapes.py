@@ -161,3 +161,31 @@ def test_gate_up_swiglu_random(cuda, seed):
     got = (act, leaves[0].grad, leaves[1].grad, leaves[2].grad)
     errs = {k: on.rel_err(np64(gv), wv) for k, gv, wv in zip(("act", "dx", "dwg", "dwu"), got, want)}
     assert all(e <= 2e-2 for e in errs.values()), errs
+
+
+@pytest.mark.parametrize("seed", _seeds(6))
+def test_gate_up_swiglu_random_wide(cuda, seed):
+    """Wider rows than the sweep above: several tiles along D and H, K splits of
+    both backward products, odd sizes among them; against float64."""
+    rng = np.random.default_rng(5000 + seed)
+    m = int(rng.integers(1, 3001))
+    d = int(rng.integers(321, 1500))
+    h = int(rng.integers(100, 3000))
+    if seed % 2 == 0:  # rows of whole vectors
+        d, h = d // 8 * 8, h // 8 * 8
+    note(f"gemm swiglu random wide seed={seed} m={m} d={d} h={h}")
+    g = gen(seed)
+    x = randn((m, d), g, torch.bfloat16, cuda)
+    wg = randn((h, d), g, torch.bfloat16, cuda, std=d ** -0.5)
+    wu = randn((h, d), g, torch.bfloat16, cuda, std=d ** -0.5)
+    dact = randn((m, h), g, torch.bfloat16, cuda)
+    leaves = [t.detach().requires_grad_(True) for t in (x, wg, wu)]
+    act = fused_gate_up_swiglu(*leaves)
+    got = [act, *torch.autograd.grad(act, leaves, dact)]
+    exact = [t.double().requires_grad_(True) for t in (x, wg, wu)]
+    e = torch.nn.functional.silu(exact[0] @ exact[1].T) * (exact[0] @ exact[2].T)
+    want = [e, *torch.autograd.grad(e, exact, dact.double())]
+    # at most four bf16 roundings in a row (a and b, da and db, the result):
+    # 2^-9 of each value at most
+    for v, w in zip(got, want):
+        assert (v.double() - w).norm() <= 4 * 2.0 ** -9 * w.norm()
