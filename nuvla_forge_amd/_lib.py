@@ -140,9 +140,10 @@ def native():
 
 
 def available() -> bool:
-    """True if libnf_hip.so loads (it may still lack a GPU to run on)."""
+    """True if libnf_hip.so and the ops' host side in _native.so load: what a call
+    on device tensors needs (there may still be no GPU to run on)."""
     try:
-        lib()
+        native()  # loads the product library first
         return True
     except RuntimeError:
         return False

@@ -153,3 +153,30 @@ def test_native_route_leaves_host_and_meta_tensors_alone():
         assert n.ce(t, t, i, 16, -100, 1) is None
     assert n.swiglu(a, None) is None and n.swiglu(a) is None
     assert n.seam(a, a, a, a[0], a, a, 1, "eps") is None
+
+
+def test_without_the_extension_module_the_fused_path_is_not_usable():
+    """HAS_TRITON / HAS_HIP say whether a device call would run: it needs the
+    C++ host side beside the product library, and raises without it."""
+    import subprocess
+    import sys
+    from pathlib import Path
+
+    code = """
+import sys
+sys.modules["nuvla_forge_amd._native"] = None  # its import raises ImportError
+from nuvla_forge_amd import _lib, kernels
+_lib.lib()
+assert not kernels.HAS_TRITON and not kernels.utils.HAS_HIP and not _lib.available()
+try:
+    _lib.native()
+except RuntimeError as e:
+    assert "_native.so" in str(e)
+else:
+    raise AssertionError("no error")
+"""
+    run = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True,
+                         cwd=Path(__file__).resolve().parents[1])
+    assert run.returncode == 0, run.stderr
+    from nuvla_forge_amd import _lib, kernels
+    assert _lib.available() and kernels.utils.HAS_HIP
