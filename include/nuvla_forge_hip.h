@@ -185,9 +185,10 @@ int nf_adaln_bwd_reduce(void *workspace, size_t workspace_bytes,
 
 /* The whole adaLN seam backward in one call: the results of nf_adaln_bwd and
  * nf_adaln_bwd_reduce (same arguments, outputs each NULL where not wanted),
- * with a workspace of nf_adaln_bwd_workspace(M, N, T) bytes.  With many
- * samples it runs without partial rows per sample (the sums differ from the
- * two calls' by fp32 rounding only); fixed orders, no atomics. */
+ * with a workspace of nf_adaln_bwd_workspace(M, N, T) bytes.  Over many
+ * samples of N <= 4096 it mostly runs without partial rows per sample (the
+ * sums differ from the two calls' by fp32 rounding only); fixed orders, no
+ * atomics. */
 int nf_adaln_bwd_full(const void *dh_up, const void *dout, const void *x,
                       int64_t ld_x, const void *y, int64_t ld_y,
                       const void *gate, int64_t ld_gate, const void *weight,

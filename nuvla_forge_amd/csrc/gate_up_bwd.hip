@@ -16,8 +16,8 @@
 // chip together.
 //
 // Each product may be split along K into S fp32 slices added in order by
-// gate_up_reduce_kernel; make_plan picks the splits.  Encoder MLP (M 9408 D 384
-// H 1536) and M 4096 D 2048 H 5632: see make_plan.
+// gate_up_reduce_kernel; pick_split picks the splits.  Large bf16 products keep
+// the earlier form: nf_gemm_swiglu_bwd_wins.
 #include "gemm_store.h"
 
 namespace nf {
