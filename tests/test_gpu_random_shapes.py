@@ -189,3 +189,31 @@ def test_gate_up_swiglu_random_wide(cuda, seed):
     # 2^-9 of each value at most
     for v, w in zip(got, want):
         assert (v.double() - w).norm() <= 4 * 2.0 ** -9 * w.norm()
+
+
+@pytest.mark.parametrize("seed", _seeds(8))
+def test_ce_random_wide(cuda, seed):
+    """Larger extents than the sweep above: V and M on both sides of 4096, where
+    rows start to be padded to lines, several chunks, tiles of 192 and 256 along D,
+    K splits of dH; against float64."""
+    rng = np.random.default_rng(6000 + seed)
+    m, v = int(rng.integers(200, 7000)), int(rng.integers(1000, 12000))
+    d = int(rng.integers(100, 700)) if seed % 2 else int(rng.integers(16, 90)) * 8
+    chunk = int(rng.integers(64, 3000))
+    dt = _pick(rng, DT[:2])
+    frac = float(rng.random()) * 0.5
+    note(f"ce random wide seed={seed} m={m} d={d} v={v} chunk={chunk} ignore={frac:.2f} dt={dt}")
+    g = gen(seed)
+    leaves = [randn((m, d), g, dt, cuda).requires_grad_(True),
+              randn((v, d), g, dt, cuda, std=2.0 * d ** -0.5).requires_grad_(True)]
+    tgt = torch.randint(0, v, (m,), generator=g)
+    tgt[torch.rand(m, generator=g) < frac] = -100
+    tgt = tgt.to(cuda)
+    loss = chunked_cross_entropy(*leaves, tgt, chunk_size=chunk)
+    got = torch.autograd.grad(loss, leaves)
+    exact = [t.detach().double().requires_grad_(True) for t in leaves]
+    want = torch.nn.functional.cross_entropy(exact[0] @ exact[1].T, tgt)
+    grads = torch.autograd.grad(want, exact)
+    assert abs(float(loss.detach()) - float(want.detach())) <= TOL[dt] * float(want.detach())
+    for a, e in zip(got, grads):
+        assert (a.double() - e).norm() <= TOL[dt] * e.norm()

@@ -332,3 +332,25 @@ def test_gate_up_fwd_bwd_replays_in_a_graph(cuda):
         return step
 
     assert_graph_replays_match(make)
+
+
+def test_gate_up_large_fwd_bwd_replays_in_a_graph(cuda):
+    """The same for products above the line of nf_gemm_swiglu_bwd_wins, whose dx
+    is two library GEMMs."""
+    from tests.helpers import assert_graph_replays_match
+
+    m, d, h = 2048, 4096, 8192
+    note(f"gate/up graph replay m={m} d={d} h={h}")
+    assert not _lib.lib().nf_gemm_swiglu_bwd_wins(m, d, h)
+    x, wg, wu, dact = _inputs(m, d, h, torch.bfloat16, cuda, seed=13)
+
+    def make():
+        leaves = [t.detach().requires_grad_(True) for t in (x, wg, wu)]
+
+        def step():
+            act = fused_gate_up_swiglu(*leaves)
+            return (act, *torch.autograd.grad(act, leaves, dact))
+
+        return step
+
+    assert_graph_replays_match(make)
