@@ -107,7 +107,9 @@ int nf_gemm_swiglu_wgrad(const void *da, const void *db, int64_t ld_ab,
  * dw_gate = da^T x and dw_up = db^T x ([H, D], dt_dw), contiguous, each NULL
  * where not wanted; fp32 accumulation over both terms of dx, one rounding to
  * the output type, fixed orders.  Operands, limits and M == 0 as in
- * nf_gemm_swiglu and nf_gemm_swiglu_wgrad; the operands are read as they lie.
+ * nf_gemm_swiglu and nf_gemm_swiglu_wgrad; the operands are read as they
+ * lie, or through padded copies in the workspace where D or H is no multiple of
+ * 8 (rows whose base or stride alone is off 16 bytes are read element-wise).
  * Workspace: nf_gemm_swiglu_bwd_workspace bytes (may be 0), 16-byte aligned;
  * its want flags say which outputs are not NULL. */
 size_t nf_gemm_swiglu_bwd_workspace(int64_t M, int64_t D, int64_t H,

@@ -120,8 +120,8 @@ __device__ __forceinline__ void clear(floatx16 (&acc)[C::TM][C::TN]) {
 }
 
 // BUF: rows of whole 16-byte vectors (D, H and the strides multiples of 8,
-// aligned bases): buffer copies and vector stores; else register copies and
-// element stores.
+// aligned bases): buffer copies and vector stores; else (views of other
+// alignments, padded rows past 2 GiB) register copies and element stores.
 template <bool BUF>
 __global__ NF_GEMM_BOUNDS(C) void gate_up_bwd_kernel(Args p) {
   __shared__ __attribute__((aligned(16))) char smem[C::LDS_BYTES];
@@ -221,6 +221,73 @@ __global__ __launch_bounds__(kSumThreads) void gate_up_reduce_kernel(Sums p) {
   }
 }
 
+// Rows that are not whole 16-byte vectors (D or H no multiple of 8): each tile would
+// read them two bytes at a time through registers.  So the operands are copied
+// once to rows of Dp and Hp elements, zeros past D and H, the products run on Dp
+// and Hp, into fp32 slices, and the reduce below drops the padding.  Forward +
+// backward, us, element-wise tiles -> padded: M 9408 D 383 H 1537 482 -> 274, M
+// 4096 D 2047 H 5631 2446 -> 1308, M 300 D 77 H 501 71 -> 45, M 64 D 300 H 1030
+// 75 -> 58.  Up to five matrices a launch; a block takes kSumThreads vectors of one.
+struct Pad {
+  const bf16 *in;
+  bf16 *out;
+  int64_t rows, cols, ld;  // what is there
+  int64_t ld_out;          // elements a padded row
+  int64_t vectors, blocks; // of the padded rows
+};
+struct Pads {
+  Pad j[5];
+  int n;
+};
+static __global__ __launch_bounds__(kSumThreads) void gate_up_pad_kernel(Pads p) {
+  int64_t b = blockIdx.x;
+  int k = 0;
+  while (k < p.n - 1 && b >= p.j[k].blocks) b -= p.j[k++].blocks;
+  const Pad &q = p.j[k];
+  const int64_t v = b * kSumThreads + threadIdx.x;
+  if (v >= q.vectors) return;
+  const int64_t vpr = q.ld_out / 8, r = v / vpr, c = (v - r * vpr) * 8;
+  const bf16 *src = q.in + r * q.ld + c;
+  bf16 e[8];
+#pragma unroll
+  for (int i = 0; i < 8; ++i)
+    e[i] = r < q.rows && c + i < q.cols ? src[i] : static_cast<bf16>(0.f);
+  u32x4 w;
+  __builtin_memcpy(&w, e, 16);
+  *reinterpret_cast<u32x4 *>(q.out + v * 8) = w;
+}
+
+// out[r, c] = the sum of the S slices at (r, c) of their rows of `pitch`, r < rows,
+// c < cols; up to three products, as above.
+struct PadSum {
+  const float *part;
+  void *out;
+  int64_t rows, cols, pitch, slice;
+  int S, dt;
+  int64_t blocks;
+};
+struct PadSums {
+  PadSum j[3];
+  int n;
+};
+static __global__ __launch_bounds__(kSumThreads) void gate_up_pad_reduce_kernel(PadSums p) {
+  int64_t b = blockIdx.x;
+  int k = 0;
+  while (k < p.n - 1 && b >= p.j[k].blocks) b -= p.j[k++].blocks;
+  const PadSum &q = p.j[k];
+  const int64_t v = b * kSumThreads + threadIdx.x, vpr = q.pitch / 4;
+  const int64_t r = v / vpr, c = (v - r * vpr) * 4;
+  if (r >= q.rows) return;
+  float a[4] = {0.f, 0.f, 0.f, 0.f};
+  for (int s = 0; s < q.S; ++s) {
+    const float4 x = *reinterpret_cast<const float4 *>(q.part + s * q.slice + v * 4);
+    a[0] += x.x; a[1] += x.y; a[2] += x.z; a[3] += x.w;
+  }
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+    if (c + i < q.cols) store_dyn(q.out, q.dt, r * q.cols + c + i, a[i]);
+}
+
 // K splits of the launch.  nx dx tiles of kx stages and nw dW tiles of kw
 // stages run on 256 CUs, one block each, the longer blocks first; a block
 // also costs ~4 stages of prologue and epilogue, and a split product the
@@ -253,9 +320,19 @@ inline Split pick_split(int64_t M, int64_t D, int64_t H, bool want_x, int want_w
   return best;
 }
 
+// rows x ld elements of 2 bytes stay under 2 GiB (32-bit buffer offsets)
+inline bool under_2gib(int64_t rows, int64_t ld) {
+  const int64_t lim = (((int64_t)1 << 31) - 64) / 2;
+  return rows >= 0 && ld > 0 && ld <= lim && rows <= (lim - 1) / ld;
+}
+
 struct Layout {
   Split sp;
-  size_t off_x, off_g, off_u, total;
+  bool pad;        // the products run on padded copies, rows of Dp and Hp
+  int64_t Dp, Hp;  // D and H where not
+  size_t off_x, off_g, off_u;  // the products' slices
+  size_t off_da, off_db, off_xp, off_wg, off_wu;  // the copies
+  size_t total;
 };
 // A thread keeps its last shape's layout: the workspace call and the launch
 // of every step ask for the same one.
@@ -269,21 +346,75 @@ inline Layout layout(int64_t M, int64_t D, int64_t H, bool x, bool g, bool u) {
   const int want = (int)x + 2 * (int)g + 4 * (int)u;
   if (kept.M == M && kept.D == D && kept.H == H && kept.want == want) return kept.L;
   Layout L{};
-  L.sp = pick_split(M, D, H, x, (int)g + (int)u);
+  const int64_t dp = gemm::round_up(D, 8), hp = gemm::round_up(H, 8);
+  L.pad = (dp != D || hp != H) && under_2gib(M, dp) && under_2gib(M, hp) && under_2gib(hp, dp);
+  L.Dp = L.pad ? dp : D;
+  L.Hp = L.pad ? hp : H;
+  L.sp = pick_split(M, L.Dp, L.Hp, x, (int)g + (int)u);
   size_t o = 0;
   auto take = [&](size_t bytes) { const size_t at = o; o = gemm::align256(o + bytes); return at; };
-  L.off_x = take(x && L.sp.sx > 1 ? (size_t)L.sp.sx * M * D * sizeof(float) : 0);
-  L.off_g = take(g && L.sp.sw > 1 ? (size_t)L.sp.sw * H * D * sizeof(float) : 0);
-  L.off_u = take(u && L.sp.sw > 1 ? (size_t)L.sp.sw * H * D * sizeof(float) : 0);
+  auto slices = [&](bool want, int S, int64_t rows) {
+    return take(want && (S > 1 || L.pad) ? (size_t)S * rows * L.Dp * sizeof(float) : 0);
+  };
+  auto copy = [&](bool want, int64_t rows, int64_t cols) {
+    return take(L.pad && want ? (size_t)rows * cols * sizeof(bf16) : 0);
+  };
+  L.off_x = slices(x, L.sp.sx, M);
+  L.off_g = slices(g, L.sp.sw, L.Hp);
+  L.off_u = slices(u, L.sp.sw, L.Hp);
+  L.off_da = copy(x || g, M, L.Hp);
+  L.off_db = copy(x || u, M, L.Hp);
+  L.off_xp = copy(g || u, M, L.Dp);
+  L.off_wg = copy(x, L.Hp, L.Dp);
+  L.off_wu = copy(x, L.Hp, L.Dp);
   L.total = o;
   kept = {M, D, H, want, L};
   return L;
 }
 
-// rows x ld elements of 2 bytes stay under 2 GiB (32-bit buffer offsets)
-inline bool under_2gib(int64_t rows, int64_t ld) {
-  const int64_t lim = (((int64_t)1 << 31) - 64) / 2;
-  return rows >= 0 && ld > 0 && ld <= lim && rows <= (lim - 1) / ld;
+// The launch on padded copies: a holds the padded extents and the operands as they
+// lie, its jobs' slices the padded products.
+inline int launch_padded(Args a, const Layout &L, char *ws, int64_t total, void *dx, int dt_dx,
+                         void *dw_gate, void *dw_up, int dt_dw, int64_t D, int64_t H,
+                         hipStream_t s) {
+  const bool any_w = dw_gate || dw_up;
+  Pads pd{};
+  int64_t blocks = 0;
+  auto pad = [&](const bf16 *&m, size_t off, int64_t rows, int64_t cols, int64_t ld,
+                 int64_t rows_out, int64_t ld_out) {
+    bf16 *out = reinterpret_cast<bf16 *>(ws + off);
+    const int64_t vectors = rows_out * (ld_out / 8);
+    const int64_t nb = (vectors + kSumThreads - 1) / kSumThreads;
+    pd.j[pd.n++] = Pad{m, out, rows, cols, ld, ld_out, vectors, nb};
+    blocks += nb;
+    m = out;
+  };
+  if (dx || dw_gate) pad(a.da, L.off_da, a.M, H, a.ld_ab, a.M, L.Hp);
+  if (dx || dw_up) pad(a.db, L.off_db, a.M, H, a.ld_ab, a.M, L.Hp);
+  if (any_w) pad(a.x, L.off_xp, a.M, D, a.ldx, a.M, L.Dp);
+  if (dx) pad(a.wg, L.off_wg, H, D, a.ldg, L.Hp, L.Dp);
+  if (dx) pad(a.wu, L.off_wu, H, D, a.ldu, L.Hp, L.Dp);
+  a.ld_ab = L.Hp;
+  a.ldx = a.ldg = a.ldu = L.Dp;
+  PadSums q{};
+  int64_t sum_blocks = 0;
+  auto sum = [&](const Job &j, void *out, int64_t rows, int dt) {
+    if (!out) return;
+    const int64_t nb = (rows * (L.Dp / 4) + kSumThreads - 1) / kSumThreads;
+    q.j[q.n++] = PadSum{j.part, out, rows, D, L.Dp, j.rows * L.Dp, j.S, dt, nb};
+    sum_blocks += nb;
+  };
+  sum(a.dx, dx, a.M, dt_dx);
+  sum(a.dwg, dw_gate, H, dt_dw);
+  sum(a.dwu, dw_up, H, dt_dw);
+  if (blocks > 0x7fffffffLL || sum_blocks > 0x7fffffffLL)
+    return set_error(NF_ERR_ARG, "nf_gemm_swiglu_bwd: grid too large");
+  gate_up_pad_kernel<<<(unsigned)blocks, kSumThreads, 0, s>>>(pd);
+  if (int e = check_launch("gate_up_pad")) return e;
+  gate_up_bwd_kernel<true><<<(unsigned)total, C::NT, 0, s>>>(a);
+  if (int e = check_launch("nf_gemm_swiglu_bwd")) return e;
+  gate_up_pad_reduce_kernel<<<(unsigned)sum_blocks, kSumThreads, 0, s>>>(q);
+  return check_launch("gate_up_pad_reduce");
 }
 
 }  // namespace gate_up
@@ -360,8 +491,8 @@ extern "C" int nf_gemm_swiglu_bwd(const void *da, const void *db, int64_t ld_ab,
   a.wg = static_cast<const bf16 *>(w_gate);
   a.wu = static_cast<const bf16 *>(w_up);
   a.ld_ab = ld_ab; a.ldx = ldx; a.ldg = ld_gate; a.ldu = ld_up;
-  a.M = M; a.D = D; a.H = H;
-  a.tiles_d = (int)((D + C::BM - 1) / C::BM);
+  a.M = M; a.D = L.Dp; a.H = L.Hp;
+  a.tiles_d = (int)((a.D + C::BM - 1) / C::BM);
   int64_t total = 0;
   auto job = [&](void *out, size_t off, int64_t rows, int dt, int64_t K_stages, int S) {
     Job j{};
@@ -372,17 +503,22 @@ extern "C" int nf_gemm_swiglu_bwd(const void *da, const void *db, int64_t ld_ab,
     j.tiles_n = (int)((rows + C::BN - 1) / C::BN);
     j.stages = (int)((K_stages + S - 1) / S);
     j.S = (int)((K_stages + j.stages - 1) / j.stages);
+    if (L.pad && out && j.S == 1) {  // one slice: the sum's input all the same
+      j.out = j.part;
+      j.dt = NF_DTYPE_F32;
+    }
     const int64_t blocks = out ? (int64_t)a.tiles_d * j.tiles_n * j.S : 0;
     total += blocks;
     j.blocks = (int)blocks;
     return j;
   };
-  const int64_t kx = 2 * ((H + C::BK - 1) / C::BK), kw = (M + C::BK - 1) / C::BK;
+  const int64_t kx = 2 * ((a.H + C::BK - 1) / C::BK), kw = (M + C::BK - 1) / C::BK;
   a.dx = job(dx, L.off_x, M, dt_dx, kx, L.sp.sx);
-  a.dwg = job(dw_gate, L.off_g, H, dt_dw, kw, L.sp.sw);
-  a.dwu = job(dw_up, L.off_u, H, dt_dw, kw, L.sp.sw);
+  a.dwg = job(dw_gate, L.off_g, a.H, dt_dw, kw, L.sp.sw);
+  a.dwu = job(dw_up, L.off_u, a.H, dt_dw, kw, L.sp.sw);
   if (total > 0x7fffffffLL) return set_error(NF_ERR_ARG, "nf_gemm_swiglu_bwd: grid too large");
   a.first_w = a.dwg.stages > a.dx.stages;
+  if (L.pad) return launch_padded(a, L, ws, total, dx, dt_dx, dw_gate, dw_up, dt_dw, D, H, s);
   const bool buf = D % 8 == 0 && H % 8 == 0 && ld_ab % 8 == 0 && ldx % 8 == 0 &&
                    ld_gate % 8 == 0 && ld_up % 8 == 0 && aligned16(da) && aligned16(db) &&
                    aligned16(x) && aligned16(w_gate) && aligned16(w_up) && aligned16(dx) &&

@@ -151,6 +151,8 @@ class _FusedGateUpSwiGLU(torch.autograd.Function):
                     )
                     one_w = False
             if one_x or one_w:
+                if d % 8 == 0 and h % 8 == 0:  # other widths go to padded rows in the call
+                    x, w_gate, w_up = (_vector_rows(t.detach()) for t in (x, w_gate, w_up))
                 pg, pu = (_lib.ptr(dwg), _lib.ptr(dwu)) if one_w else (None, None)
                 nbytes = L.nf_gemm_swiglu_bwd_workspace(m, d, h, one_x, bool(pg), bool(pu))
                 ws = torch.empty(max(nbytes, 1), dtype=torch.uint8, device=x.device)
@@ -212,6 +214,14 @@ def _rows_bf16(t: torch.Tensor) -> torch.Tensor:
     """bf16 with unit-stride rows (a cast / copy only when needed)."""
     t = t.to(torch.bfloat16)
     return t if t.stride(-1) == 1 else t.contiguous()
+
+
+def _vector_rows(t: torch.Tensor) -> torch.Tensor:
+    """``t`` with rows of whole 16-byte vectors (its width is a multiple of 8): a
+    copy of a view whose base or row stride is not, which the backward would
+    read element by element."""
+    whole = t.data_ptr() % 16 == 0 and t.stride(0) % 8 == 0
+    return t if whole else t.clone(memory_format=torch.contiguous_format)
 
 
 def fused_swiglu(a: torch.Tensor, b: torch.Tensor, force_reference: bool = False) -> torch.Tensor:

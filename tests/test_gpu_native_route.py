@@ -160,6 +160,37 @@ def test_gate_up_gradients_in_any_input_types(cuda, xd, gd, ud, need):
     _same(got, [v.to(t) for v, t in zip(want, types)])
 
 
+@pytest.mark.parametrize("which", ["x offset", "x stride", "w_gate offset", "w_up stride", "all"])
+def test_gate_up_backward_of_views_off_vector_alignment(cuda, which):
+    """Row-strided bf16 views whose rows do not start on 16 bytes: the same bits as
+    contiguous copies of them, from both hosts."""
+    note(f"gate/up views {which}")
+    m, d, h = 300, 72, 136
+    g = gen(14)
+
+    def view(name, rows):
+        wide = randn((rows, d + 16), g, BF16, cuda, std=1.0 if name == "x" else d ** -0.5)
+        off = 1 if which in (f"{name} offset", "all") else 0
+        if which == f"{name} stride":
+            wide = wide[:, :d + 3].contiguous()
+        return wide[:, off:off + d]
+
+    inputs = [view("x", m), view("w_gate", h), view("w_up", h)]
+    assert any(v.data_ptr() % 16 or v.stride(0) % 8 for v in inputs)
+    up = [randn((m, h), g, BF16, cuda)]
+
+    def run(fn, ops):
+        leaves = [v.detach().requires_grad_(True) for v in ops]  # keeps strides
+        out = fn(*leaves)
+        return [out.detach(), *torch.autograd.grad(out, leaves, up)]
+
+    got = run(fused_gate_up_swiglu, inputs)
+    _same(got, run(swiglu._FusedGateUpSwiGLU.apply, inputs))
+    want = run(fused_gate_up_swiglu, [v.contiguous().clone() for v in inputs])
+    for a, e in zip(got[1:], want[1:]):
+        assert (a.double() - e.double()).norm() <= 2.0 ** -7 * e.double().norm()
+
+
 @pytest.mark.parametrize("need", [(True, True, True), (True, False, False), (False, True, True),
                                   (True, False, True)])
 def test_gate_up_large_products(cuda, need):

@@ -260,12 +260,15 @@ def _bwd_inputs(m, d, h, pad, dev, seed):
 # tile edges (256) and remainders, slices of dx's K across the seam between the
 # gate and the up units (an odd number of 64-deep stages each), more than 8 dx
 # slices, ragged last slices of both products, rows that are not whole vectors
-# (element-wise copies and stores), one token, one unit
+# (padded copies: a workspace for both products whether split or not), strides
+# that are not (element-wise copies and stores), one token, one unit
 @pytest.mark.parametrize("m,d,h,pad,sx,sw", [
     (256, 256, 256, 0, True, False), (257, 264, 328, 8, True, False),
     (40, 72, 4104, 0, True, False), (3000, 136, 264, 8, True, True),
-    (700, 200, 1000, 16, True, True), (300, 37, 101, 3, False, False),
-    (1100, 36, 700, 0, True, True), (1, 8, 8, 0, False, False), (513, 520, 1, 7, False, True)])
+    (700, 200, 1000, 16, True, True), (300, 37, 101, 3, True, True),
+    (1100, 36, 700, 0, True, True), (1, 8, 8, 0, False, False), (513, 520, 1, 7, True, True),
+    (257, 263, 1001, 2, True, True), (3000, 255, 257, 0, True, True), (1, 1, 1, 0, True, True),
+    (300, 72, 136, 3, False, False)])
 def test_gate_up_bwd_entry_matches_fp64(cuda, m, d, h, pad, sx, sw):
     """dx = da W_gate + db W_up, dW_gate = da^T x, dW_up = db^T x in fp32 from the
     same bf16 operands in fp64, element by element; a second call gives the
@@ -289,13 +292,14 @@ def test_gate_up_bwd_entry_matches_fp64(cuda, m, d, h, pad, sx, sw):
         assert torch.equal(v, a) and torch.equal(v.bfloat16(), b)
 
 
+@pytest.mark.parametrize("d,h", [(200, 1000), (201, 1003)])
 @pytest.mark.parametrize("want", [(True, False, False), (False, True, False), (False, False, True),
                                   (True, True, False), (False, True, True), (False, False, False)])
-def test_gate_up_bwd_entry_writes_what_is_wanted(cuda, want):
+def test_gate_up_bwd_entry_writes_what_is_wanted(cuda, want, d, h):
     """Any subset of the gradients: the values of a call for all three (their K
     split may differ: an fp32 sum in another order)."""
-    m, d, h = 700, 200, 1000
-    note(f"gate/up bwd entry subset {want}")
+    m = 700
+    note(f"gate/up bwd entry subset {want} d={d} h={h}")
     ops = _bwd_inputs(m, d, h, 0, cuda, 5)
     every, _ = _bwd(*ops, torch.float32)
     got, _ = _bwd(*ops, torch.float32, want)
