@@ -121,10 +121,11 @@ int nf_gemm_swiglu_bwd(const void *da, const void *db, int64_t ld_ab,
                        int dt_dw, int64_t M, int64_t D, int64_t H, int dtype,
                        void *workspace, size_t workspace_bytes, void *stream);
 
-/* 1 where nf_gemm_swiglu_bwd is the faster form of an all-bf16 backward that
- * wants all three gradients, 0 where nf_gemm_swiglu_wgrad beside library GEMMs
- * for dx is (large products).  Either form takes every size. */
-int nf_gemm_swiglu_bwd_wins(int64_t M, int64_t D, int64_t H);
+/* 1 where nf_gemm_swiglu_bwd is the faster form of an all-bf16 backward, 0 where
+ * library GEMMs for dx, and nf_gemm_swiglu_wgrad beside them, are (large
+ * products; sooner where want_dw says that dx alone is wanted).  Either form
+ * takes every size. */
+int nf_gemm_swiglu_bwd_wins(int64_t M, int64_t D, int64_t H, int want_dw);
 
 /* ------------------------------------------------------------------------
  * adaLN-Zero seam: gated residual add, RMSNorm, modulation.  Row m of the

@@ -76,7 +76,7 @@ SIGNATURES = {
     "nf_gemm_swiglu": (
         _I32, [_P, _I64, _P, _I64, _P, _I64, _P, _P, _P, _I64, _I64, _I64, _I64, _I32, _P],
     ),
-    "nf_gemm_swiglu_bwd_wins": (_I32, [_I64, _I64, _I64]),
+    "nf_gemm_swiglu_bwd_wins": (_I32, [_I64, _I64, _I64, _I32]),
     "nf_gemm_swiglu_bwd_workspace": (_SZ, [_I64, _I64, _I64, _I32, _I32, _I32]),
     "nf_gemm_swiglu_bwd": (
         _I32,

@@ -435,9 +435,14 @@ using namespace nf;
 //   M 8192 D 2048 H 5632 1302 / 1208; M 4096 D 4096 H 11008 2270 / 1970;
 //   M 16384 D 4096 H 5632 4398 / 3880; M 8192 D 8192 H 8192 5996 / 5202.
 // (The transposed copies, M padded to 8, must stay under 2 GiB.)
-extern "C" int nf_gemm_swiglu_bwd_wins(int64_t M, int64_t D, int64_t H) {
-  const bool large = M >= 2048 && D >= 2048 && H >= 2560 &&
-                     (double)M * (double)D * (double)H >= 6.5e10;
+// dx alone (frozen weights) has no transposes to weigh against, so the library's
+// products win sooner: M 9408 D 1000 H 2731 439 / 358, M 9408 D 384 H 1536 120 / 111,
+// M 16384 D 1536 H 4096 1042 / 904, M 4096 D 2048 H 5632 447 / 411; M 4096 D 768 H
+// 3072 144 / 153, M 2048 D 1536 H 4096 145 / 162, M 512 D 2048 H 5632 113 / 129.
+extern "C" int nf_gemm_swiglu_bwd_wins(int64_t M, int64_t D, int64_t H, int want_dw) {
+  const double work = (double)M * (double)D * (double)H;
+  if (!want_dw) return !(M >= 8192 || work >= 2.5e10);
+  const bool large = M >= 2048 && D >= 2048 && H >= 2560 && work >= 6.5e10;
   return !(large && gate_up::under_2gib(M + 7, H > D ? H : D));
 }
 

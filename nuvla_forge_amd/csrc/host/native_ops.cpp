@@ -267,7 +267,8 @@ struct GateUp : torch::autograd::Function<GateUp> {
     bool one_x = ctx->needs_input_grad(0), one_w = need_g || need_u;  // left to the one launch
     if (need_g) dg = at::empty({h, d}, x.options().dtype(tw));
     if (need_u) du = at::empty({h, d}, x.options().dtype(tw));
-    if (tx == at::kBFloat16 && tg == tx && tu == tx && !nf_gemm_swiglu_bwd_wins(m, d, h)) {
+    if (tx == at::kBFloat16 && tg == tx && tu == tx &&
+        !nf_gemm_swiglu_bwd_wins(m, d, h, one_w)) {
       if (one_x) {
         const c10::impl::ExcludeDispatchKeyGuard no_autocast(c10::autocast_dispatch_keyset);
         dx = at::addmm(at::mm(da, wg), db, wu);

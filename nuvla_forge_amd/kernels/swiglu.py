@@ -76,8 +76,9 @@ class _FusedGateUpSwiGLU(torch.autograd.Function):
     recomputed); ``nf_gemm_swiglu_bwd`` computes dx = da W_gate + db W_up,
     dW_gate = da^T x and dW_up = db^T x in one launch, each written once in
     its input's type (sums over K splits added in a fixed order).  Where
-    ``nf_gemm_swiglu_bwd_wins`` says no (large all-bf16 products), dx is two
-    library GEMMs and both weight gradients come from ``nf_gemm_swiglu_wgrad``.
+    ``nf_gemm_swiglu_bwd_wins`` says no (large all-bf16 products, sooner for dx
+    alone), dx is two library GEMMs and both weight gradients come from
+    ``nf_gemm_swiglu_wgrad``.
     """
 
     @staticmethod
@@ -135,7 +136,8 @@ class _FusedGateUpSwiGLU(torch.autograd.Function):
         one_x, one_w = need_x, need_g or need_u  # left to the one launch
         with device_of(x):
             st = _lib.stream_of(x)
-            if tx == tg == tu == torch.bfloat16 and not L.nf_gemm_swiglu_bwd_wins(m, d, h):
+            if (tx == tg == tu == torch.bfloat16
+                    and not L.nf_gemm_swiglu_bwd_wins(m, d, h, one_w)):
                 if one_x:
                     with torch.no_grad(), torch.autocast(x.device.type, enabled=False):
                         dx = torch.addmm(torch.mm(da, w_gate), db, w_up)

@@ -213,7 +213,14 @@ def test_gemm_swiglu_bwd_workspace_and_validation():
     ((1 << 17) - 3, 2048, 8192, 1),         # ... and the padded copies no longer
     (0, 4096, 4096, 1)])
 def test_gemm_swiglu_bwd_wins_where_it_was_measured_to(m, d, h, wins):
-    assert _lib.lib().nf_gemm_swiglu_bwd_wins(m, d, h) == wins
+    assert _lib.lib().nf_gemm_swiglu_bwd_wins(m, d, h, 1) == wins
+
+
+@pytest.mark.parametrize("m,d,h,wins", [
+    (9408, 384, 1536, 0), (8192, 256, 512, 0), (8191, 256, 512, 1), (4096, 768, 3072, 1),
+    (4096, 2048, 5632, 0), (2048, 1536, 4096, 1), (512, 2048, 5632, 1)])
+def test_gemm_swiglu_bwd_wins_for_dx_alone(m, d, h, wins):
+    assert _lib.lib().nf_gemm_swiglu_bwd_wins(m, d, h, 0) == wins
 
 
 def test_adaln_argument_validation():

@@ -345,7 +345,7 @@ def test_gate_up_large_fwd_bwd_replays_in_a_graph(cuda):
 
     m, d, h = 2048, 4096, 8192
     note(f"gate/up graph replay m={m} d={d} h={h}")
-    assert not _lib.lib().nf_gemm_swiglu_bwd_wins(m, d, h)
+    assert not _lib.lib().nf_gemm_swiglu_bwd_wins(m, d, h, 1)
     x, wg, wu, dact = _inputs(m, d, h, torch.bfloat16, cuda, seed=13)
 
     def make():
